@@ -309,9 +309,8 @@ class Session:
         check(lib().ifem_gpu_assemble(self.h, C.byref(s), ngv, precision))
 
     def autotune_assembly(self, itg, ng, precision: int = FP64) -> int:
-        """Pick the fastest element-chunk variant for this system; returns 0
-        for full chunks, 1 for half chunks, 2 for full chunks in two
-        Gauss-point slabs.  K and b are left as after assemble()."""
+        """Pick the fastest work split of the line kernels for this system;
+        returns the variant as in set_assembly_variant.  K and b are left as after assemble()."""
         keep = []
         s = self._integrand(itg, keep)
         ngv = (C.c_int * 3)(*ng)
@@ -320,8 +319,8 @@ class Session:
         return h.value
 
     def set_assembly_variant(self, p, ng, ncomp, precision, variant):
-        """Fix the element-chunk variant for (p, ng, ncomp, precision); -1
-        restores the built-in default."""
+        """Fix the work split (0, 1 or 2, see ifem_gpu_set_assembly_variant)
+        for (p, ng, ncomp, precision); -1 restores the built-in choice."""
         check(lib().ifem_gpu_set_assembly_variant(self.h, p, ng, ncomp, precision, variant))
 
     def norms(self, itg, ng, exact=None):

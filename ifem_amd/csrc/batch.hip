@@ -295,7 +295,7 @@ void Batch::release()
     graph_check[g] = 0;
   }
   ready = fp64_ready = fp32_ready = tuned = geo_valid = false;
-  neq = nitems = nchunk = 0;
+  neq = nchunk = 0;
   nnz = ngp = 0;
   h_gp0.clear();
   for (int p = 0; p < 4; p++) {
@@ -617,8 +617,8 @@ int batch_solve(Context& c, const ifem_gpu_solver_params& prm, ifem_gpu_stats* s
   return IFEM_GPU_OK;
 }
 
-// Autotuner: for each degree present, the element-chunk variant of the
-// assembly (full or half chunk) and the SpMV lanes per row (16, 32, 64),
+// Autotuner: for each degree present, the work split of the assembly (row
+// segments of full or half length) and the SpMV lanes per row (16, 32, 64),
 // each chosen by timing the whole batch with the other degrees fixed.
 int batch_autotune(Context& c, int precision, int* table)
 {
@@ -632,8 +632,6 @@ int batch_autotune(Context& c, int precision, int* table)
     int best_half = 0;
     for (int half = 0; half <= 1; half++) {
       B.tune[p].half = half;
-      rc = batch_upload_args(c);
-      if (rc) return rc;
       double t = 1e300;
       for (int rep = 0; rep < 2; rep++) {
         double ms = 0.0;
@@ -648,9 +646,7 @@ int batch_autotune(Context& c, int precision, int* table)
     }
     B.tune[p].half = best_half;
   }
-  rc = batch_upload_args(c);
-  if (rc) return rc;
-  // re-assemble with the chosen variants (their summation orders differ)
+  // leave the batch assembled with the chosen variants
   if (B.fp64_ready || precision == IFEM_GPU_FP64) {
     rc = batch_assemble(c, IFEM_GPU_FP64, nullptr);
     if (rc) return rc;

@@ -25,8 +25,8 @@ struct BatchPatch {
   double* span[3] = {nullptr, nullptr, nullptr};
 };
 
-// Per-degree tuning: element-chunk variant of the assembly and lanes per row
-// of the SpMV.
+// Per-degree tuning: work list of the assembly (half: segments of half the
+// length) and lanes per row of the SpMV.
 struct BatchTune {
   int half = 0;
   int lanes = 0; // 0: by row length
@@ -52,9 +52,8 @@ struct Batch {
   // assembly work list and per-patch arguments (AsmArgs, FP64 and FP32)
   void* d_args64 = nullptr;
   void* d_args32 = nullptr;
-  int2* d_items = nullptr;
-  int nitems = 0;
-  int item0[4] = {0, 0, 0, 0}, item1[4] = {0, 0, 0, 0}; // items of degree p: [item0[p], item1[p])
+  void* d_items = nullptr; // LineItem; of degree p in list h: [item0[h][p], item1[h][p])
+  int item0[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}}, item1[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
   int* d_queue = nullptr;   // one queue counter per degree
   int ncu = 0;              // compute units (persistent grid size)
   // geometry records per (element, Gauss point) (patch q's records start at

@@ -166,20 +166,22 @@ int ifem_gpu_assemble(ifem_gpu_ctx* ctx, const ifem_gpu_integrand* itg,
                       const int ng[3], int precision);
 
 /* No counterpart in the reference (part of this library's autotuner): times
- * the line-assembly kernel of the bound system with each element-chunk
- * variant (tile shape of the (p, nen) kernel: LDS per block against blocks
- * per CU): 0 full chunks, 1 half chunks, 2 full chunks with the Gauss points
- * in two slabs (p <= 2 with at most 3 points per direction: three blocks per
- * CU), keeps the fastest for this (p, ng, ncomp, precision) in the context
- * and leaves the system assembled as ifem_gpu_assemble does (apply Neumann
- * loads afterwards).  *half (may be NULL) receives the choice. */
+ * the assembly of the bound system with each work split of the line kernels,
+ * keeps the fastest for this (p, ng, ncomp, precision) in the context and
+ * leaves the system assembled as ifem_gpu_assemble does (apply Neumann loads
+ * afterwards).  Variants: 0 and 1 as below, 2 (p <= 2 with at most 3 points
+ * per direction).  *half (may be NULL) receives the choice. */
 int ifem_gpu_autotune_assembly(ifem_gpu_ctx* ctx, const ifem_gpu_integrand* itg,
                                const int ng[3], int precision, int* half);
 
-/* No counterpart in the reference: fix the element-chunk variant (as above;
- * -1 restores the built-in default) of the line kernel for (p, ng, ncomp,
- * precision) in this context.  EUNSUPPORTED for a variant that does not
- * exist for that degree and rule. */
+/* No counterpart in the reference: fix the work split of the line kernels for
+ * (p, ng, ncomp, precision) in this context; -1 restores the built-in
+ * choice.  p = 1, and p = 2 with ng = 3: 0 splits the node lines into row
+ * segments by a built-in rule, 1 into twice as many, 2 not at all (FP32
+ * elasticity at p = 2: as follows, and 2 full chunks in two Gauss-point
+ * slabs); the other degrees and rules: 0 full element chunks, 1 half chunks.
+ * EUNSUPPORTED for
+ * a variant that does not exist for that degree and rule. */
 int ifem_gpu_set_assembly_variant(ifem_gpu_ctx* ctx, int p, int ng, int ncomp, int precision,
                                   int variant);
 

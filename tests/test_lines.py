@@ -1,0 +1,57 @@
+"""Line kernels of the volume assembly (GPU): K and b against the oracle at
+the sizes where their work split can go wrong -- one element per direction,
+line groups of full and partial size, row segments of a long line, rows with
+full and with compacted windows.
+
+Tolerances: the sums are a few hundred to a few thousand products long, so
+1e-12 of the largest entry in FP64; FP32 values to 1e-5 of it."""
+import numpy as np
+import pytest
+
+import oracle
+from ifem_amd import FP32, FP64, Session
+from ifem_amd import model as M
+from ifem_amd import problems
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(1, 1, 1), (1, 8, 2), (3, 11, 1), (29, 4, 3), (64, 2, 2), (9, 22, 5)]
+
+
+def _problem(nc, p, nel, fix):
+    P = M.cube_patch(p, list(nel), 0.1, seed=p + nc)
+    if fix == "random":
+        msc = np.where(M.uniform(77, P.nnod * nc) < 0.7, 1, 0).astype(np.int32)
+    else:
+        msc = M.face_status(P, nc, [0, 0, 0, 0, 0, 0] if fix == "none" else [7, 0, 0, 1, 0, 0])
+    meqn, neq = M.equation_numbers(msc)
+    if nc == 3:
+        itg = M.Integrand(M.ELASTICITY, E=1.3, nu=0.28, body=(0.2, -0.1, 0.3))
+    else:
+        itg = M.Integrand(M.POISSON, kappa=M.lognormal_conductivity(3, 0.7, 0.3, 8),
+                          source=M.smooth_source(4, 4))
+    return problems.Problem("lines", P, itg, (p + 1,) * 3, meqn, neq)
+
+
+@pytest.mark.parametrize("fix", ["none", "faces", "random"])
+@pytest.mark.parametrize("nel", SIZES, ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("nc,p", [(1, 1), (1, 2), (3, 1), (3, 2)])
+def test_lines_match_oracle(nc, p, nel, fix):
+    if nc == 3 and nel[0] * nel[1] * nel[2] > 400:
+        nel = (nel[0], nel[1] // 2, nel[2])
+    pb = _problem(nc, p, nel, fix)
+    print(f"[gpu] lines nc={nc} p={p} nel={nel} fix={fix} neq={pb.neq}", flush=True)
+    if pb.neq == 0:
+        pytest.skip("no free DOF")
+    rp, ci, A, b = oracle.system(pb.patch, pb.integrand, pb.ng, pb.meqn, pb.neq, None, 0)
+    with Session() as s:
+        s.bind(s.add_patch(pb.patch), nc, pb.meqn, pb.neq)
+        s.init_assembly()
+        s.assemble(pb.integrand, pb.ng, FP64)
+        grp, gci, gA, gb = s.system()
+        s.assemble(pb.integrand, pb.ng, FP32)
+        A32 = s.values_fp32().astype(np.float64)
+    assert np.array_equal(grp, rp) and np.array_equal(gci, ci)
+    assert np.max(np.abs(gA - A)) <= 1e-12 * np.max(np.abs(A))
+    assert np.max(np.abs(gb - b)) <= 1e-12 * max(np.max(np.abs(b)), 1e-300)
+    assert np.max(np.abs(A32 - A)) <= 1e-5 * np.max(np.abs(A))
