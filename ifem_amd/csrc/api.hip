@@ -69,6 +69,7 @@ static void free_system(Context& c)
   hipFree(c.d_colind);
   hipFree(c.d_bcol);
   c.d_bcol = nullptr;
+  c.shapes.release();
   hipFree(c.d_val);
   hipFree(c.d_val32);
   hipFree(c.d_rhs);

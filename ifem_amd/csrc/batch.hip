@@ -26,6 +26,7 @@
 
 #include "devutil.hpp"
 #include "internal.hpp"
+#include "spmv.hpp"
 
 namespace ifem {
 
@@ -33,19 +34,20 @@ constexpr int kChunkRows = kThreads; // rows per solver chunk
 constexpr int kBS = 8;               // per-patch scalar stride (Scal slots)
 
 // ---------------------------------------------------------------------------
-template <typename V, typename ACC, int L, bool DOT>
+// SHAPED: columns from the row shapes (start per row, table `colind`).
+template <typename V, typename ACC, int L, bool DOT, bool SHAPED>
 __device__ inline double bspmv_rows(int r0, int r1, const int64_t* __restrict__ rowptr,
+                                    const int32_t* __restrict__ start,
                                     const int32_t* __restrict__ colind, const V* __restrict__ val,
                                     const V* __restrict__ p, V* __restrict__ q)
 {
   const int g = threadIdx.x / L, l = threadIdx.x % L;
   double pq = 0.0;
   for (int row = r0 + g; row < r1; row += kThreads / L) {
-    const int64_t b = rowptr[row], e = rowptr[row + 1];
-    ACC s = 0;
-    for (int64_t k = b + l; k < e; k += L) s += (ACC)val[k] * (ACC)p[colind[k]];
-#pragma unroll
-    for (int off = L / 2; off >= 1; off >>= 1) s += __shfl_xor(s, off, L);
+    const int64_t b = rowptr[row];
+    const int cnt = (int)(rowptr[row + 1] - b);
+    const int32_t* __restrict__ ci = SHAPED ? colind + start[row] : colind + b;
+    const ACC s = group_sum<L>(row_dot<L, ACC>(l, cnt, val + b, ci, SHAPED ? p + row : p));
     if (l == 0) {
       q[row] = (V)s;
       if (DOT) pq += (double)((ACC)p[row] * s);
@@ -55,13 +57,16 @@ __device__ inline double bspmv_rows(int r0, int r1, const int64_t* __restrict__ 
 }
 
 // q = A p over one chunk per block (lanes per row chosen per chunk); with
-// DOT, per-chunk partial <p,q> and converged patches are skipped.
-template <typename V, typename ACC, bool DOT>
+// DOT, per-chunk partial <p,q> and converged patches are skipped.  Bound by
+// the reading of the values: 400 -> 201 us per call over a solve of 48
+// diffusion patches of degrees 1 to 3 (8^3 to 36^3 elements) by the row shapes
+// and 8 instead of 64 lanes per row.
+template <typename V, typename ACC, bool DOT, bool SHAPED>
 __global__ __launch_bounds__(kThreads) void k_bspmv(
     const int* __restrict__ crow0, const int* __restrict__ cpatch, const int* __restrict__ clanes,
-    const int64_t* __restrict__ rowptr, const int32_t* __restrict__ colind,
-    const V* __restrict__ val, const V* __restrict__ p, V* __restrict__ q,
-    double* __restrict__ part_pq, const double* __restrict__ pscal)
+    const int64_t* __restrict__ rowptr, const int32_t* __restrict__ start,
+    const int32_t* __restrict__ colind, const V* __restrict__ val, const V* __restrict__ p,
+    V* __restrict__ q, double* __restrict__ part_pq, const double* __restrict__ pscal)
 {
   const int c = blockIdx.x;
   const int pt = cpatch[c];
@@ -70,9 +75,9 @@ __global__ __launch_bounds__(kThreads) void k_bspmv(
   const int r0 = crow0[c], r1 = crow0[c + 1];
   double pq;
   switch (clanes[c]) {
-  case 16: pq = bspmv_rows<V, ACC, 16, DOT>(r0, r1, rowptr, colind, val, p, q); break;
-  case 32: pq = bspmv_rows<V, ACC, 32, DOT>(r0, r1, rowptr, colind, val, p, q); break;
-  default: pq = bspmv_rows<V, ACC, 64, DOT>(r0, r1, rowptr, colind, val, p, q); break;
+  case 16: pq = bspmv_rows<V, ACC, 8, DOT, SHAPED>(r0, r1, rowptr, start, colind, val, p, q); break;
+  case 32: pq = bspmv_rows<V, ACC, 16, DOT, SHAPED>(r0, r1, rowptr, start, colind, val, p, q); break;
+  default: pq = bspmv_rows<V, ACC, 32, DOT, SHAPED>(r0, r1, rowptr, start, colind, val, p, q); break;
   }
   if (!DOT) return;
   const double bs = block_sum<double>(pq, sh);
@@ -287,6 +292,7 @@ void Batch::release()
     hipFree(*v);
     *v = nullptr;
   }
+  shapes.release();
   if (h_pscal) hipHostFree(h_pscal);
   h_pscal = nullptr;
   for (int g = 0; g < 2; g++) {
@@ -304,19 +310,19 @@ void Batch::release()
   }
 }
 
-static int default_lanes(int p)
-{
-  // interior row lengths (2p+1)^3: 27, 125, 343
-  return p <= 1 ? 16 : 64;
-}
+// Entries of a row per step: a few lanes with several steps each in flight
+// read rows of every degree best.  48 diffusion patches of degrees 1 to 3
+// (8^3 to 36^3 elements), assembly and 192 iterations: 58.8 ms with 16, 61.0
+// with 32, 67 to 79 with 64 at degree 3.
+constexpr int kLanes = 16;
 
 static int upload_lanes(Context& c)
 {
   Batch& B = *c.batch;
-  std::vector<int> lanes(B.nchunk > 0 ? B.nchunk : 1, 64);
+  std::vector<int> lanes(B.nchunk > 0 ? B.nchunk : 1, kLanes);
   for (int ch = 0; ch < B.nchunk; ch++) {
     const int p = B.pp[B.h_cpatch[ch]].p;
-    lanes[ch] = B.tune[p].lanes > 0 ? B.tune[p].lanes : default_lanes(p);
+    lanes[ch] = B.tune[p].lanes > 0 ? B.tune[p].lanes : kLanes;
   }
   IFEM_HIP(hipMemcpy(B.d_clanes, lanes.data(), sizeof(int) * lanes.size(), hipMemcpyHostToDevice));
   return IFEM_GPU_OK;
@@ -367,6 +373,8 @@ static int batch_solver_setup(Context& c)
   B.iters.assign(np, 0);
   B.conv.assign(np, 0);
   B.relres.assign(np, 0.0);
+  rc = build_row_shapes(c.stream, B.neq, B.d_rowptr, B.d_colind, false, B.nnz, B.shapes);
+  if (rc) return rc;
   IFEM_HIP(hipStreamSynchronize(c.stream));
   return IFEM_GPU_OK;
 }
@@ -376,9 +384,14 @@ static void launch_bspmv(Context& c, const V* val, const V* p, V* q)
 {
   Batch& B = *c.batch;
   if (B.nchunk == 0) return;
-  k_bspmv<V, ACC, DOT><<<B.nchunk, kThreads, 0, c.stream>>>(B.d_crow0, B.d_cpatch, B.d_clanes,
-                                                            B.d_rowptr, B.d_colind, val, p, q,
-                                                            B.part, B.pscal);
+  if (B.shapes.start)
+    k_bspmv<V, ACC, DOT, true><<<B.nchunk, kThreads, 0, c.stream>>>(
+        B.d_crow0, B.d_cpatch, B.d_clanes, B.d_rowptr, B.shapes.start, B.shapes.table, val, p, q,
+        B.part, B.pscal);
+  else
+    k_bspmv<V, ACC, DOT, false><<<B.nchunk, kThreads, 0, c.stream>>>(
+        B.d_crow0, B.d_cpatch, B.d_clanes, B.d_rowptr, nullptr, B.d_colind, val, p, q, B.part,
+        B.pscal);
 }
 
 static int read_pscal(Context& c)
@@ -618,7 +631,7 @@ int batch_solve(Context& c, const ifem_gpu_solver_params& prm, ifem_gpu_stats* s
 }
 
 // Autotuner: for each degree present, the work split of the assembly (row
-// segments of full or half length) and the SpMV lanes per row (16, 32, 64),
+// segments of full or half length) and the SpMV entries of a row per step (16, 32, 64),
 // each chosen by timing the whole batch with the other degrees fixed.
 int batch_autotune(Context& c, int precision, int* table)
 {
@@ -659,7 +672,7 @@ int batch_autotune(Context& c, int precision, int* table)
   for (int p = 1; p <= 3; p++) {
     if (!present[p]) continue;
     double best = 1e300;
-    int best_l = default_lanes(p);
+    int best_l = kLanes;
     for (int L : lanes_c) {
       B.tune[p].lanes = L;
       rc = upload_lanes(c);
@@ -689,7 +702,7 @@ int batch_autotune(Context& c, int precision, int* table)
   if (table)
     for (int p = 0; p < 4; p++) {
       table[2 * p] = B.tune[p].half;
-      table[2 * p + 1] = B.tune[p].lanes > 0 ? B.tune[p].lanes : (p > 0 ? default_lanes(p) : 0);
+      table[2 * p + 1] = B.tune[p].lanes > 0 ? B.tune[p].lanes : (p > 0 ? kLanes : 0);
     }
   return IFEM_GPU_OK;
 }

@@ -25,11 +25,19 @@ struct BatchPatch {
   double* span[3] = {nullptr, nullptr, nullptr};
 };
 
+// Row shapes of a sparsity pattern (shapes.hip): row r's k-th column is
+// r + table[start[r] + k]; start == nullptr: not available.
+struct RowShapes {
+  int32_t* start = nullptr;
+  int32_t* table = nullptr;
+  void release();
+};
+
 // Per-degree tuning: work list of the assembly (half: segments of half the
-// length) and lanes per row of the SpMV.
+// length) and row entries per step of the SpMV.
 struct BatchTune {
   int half = 0;
-  int lanes = 0; // 0: by row length
+  int lanes = 0; // 0: the default
 };
 
 struct Batch {
@@ -48,6 +56,7 @@ struct Batch {
   double* d_val = nullptr;
   float* d_val32 = nullptr;
   double* d_rhs = nullptr;
+  RowShapes shapes;
 
   // assembly work list and per-patch arguments (AsmArgs, FP64 and FP32)
   void* d_args64 = nullptr;

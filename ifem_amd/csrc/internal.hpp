@@ -149,6 +149,7 @@ struct Context {
   int64_t* d_rowptr = nullptr;
   int32_t* d_colind = nullptr;
   int32_t* d_bcol = nullptr;    // node-triple column index (3-comp, node-uniform)
+  RowShapes shapes;             // of d_bcol where that is set, else of d_colind
   double* d_val = nullptr;
   float* d_val32 = nullptr;
   double* d_rhs = nullptr;
@@ -237,6 +238,11 @@ int batch_assemble(Context& c, int precision, double* ms);
 int batch_init(Context& c);
 int batch_solve(Context& c, const ifem_gpu_solver_params& prm, ifem_gpu_stats* st);
 int batch_autotune(Context& c, int precision, int* table);
+
+// shapes.hip: row shapes of n rows (nodal: node triples, cols = node columns,
+// rowptr per equation) with `entries` column indices in all
+int build_row_shapes(hipStream_t s, int n, const int64_t* rowptr, const int32_t* cols, bool nodal,
+                     int64_t entries, RowShapes& out);
 
 // solver.hip
 int solver_setup(Context& c);

@@ -30,30 +30,37 @@
 
 #include "devutil.hpp"
 #include "internal.hpp"
+#include "spmv.hpp"
 
 namespace ifem {
 
 // ---------------------------------------------------------------------------
-// SpMV q = A p (CSR), LANES lanes per row; with DOT, per-block partial <p,q>.
+// SpMV q = A p (CSR), 8 lanes per row; with DOT, per-block partial <p,q>.
 // SKIP: return at once when scal[S_DONE] is set (work queued past convergence).
 // VV: type of the stored values (V, or FP16 values scaled by 1/scale).
-template <typename V, typename ACC, int LANES, bool DOT, bool SKIP = DOT, typename VV = V>
+// SHAPED: columns from the row shapes (start per row, table `cols`).
+// Bound by the reading of the values.  8 lanes of two entries and four steps
+// ahead take a row of 125 in one round with three butterfly steps; one wave
+// per row spent its time in the six steps of its sum and waited for two loads
+// at a time.  Diffusion 48^3 p = 2 FP64 (14.5 M entries, resident in the last
+// level cache): 29.3 -> 20 us, of which the shapes' 8 B per entry instead of
+// 12 give a third.
+template <typename V, typename ACC, bool DOT, bool SKIP = DOT, typename VV = V, bool SHAPED = false>
 __global__ __launch_bounds__(kThreads) void k_spmv_dot(
-    int n, const int64_t* __restrict__ rowptr, const int32_t* __restrict__ colind,
-    const VV* __restrict__ val, const V* __restrict__ p, V* __restrict__ q,
-    double* __restrict__ part_pq, const double* __restrict__ scal, ACC scale)
+    int n, const int64_t* __restrict__ rowptr, const int32_t* __restrict__ start,
+    const int32_t* __restrict__ cols, const VV* __restrict__ val, const V* __restrict__ p,
+    V* __restrict__ q, double* __restrict__ part_pq, const double* __restrict__ scal, ACC scale)
 {
   if (SKIP && scal[S_DONE] != 0.0) return;
   __shared__ double sh[kThreads / 64];
-  const int groups_per_block = kThreads / LANES;
-  const int g = threadIdx.x / LANES, l = threadIdx.x % LANES;
+  constexpr int L = 8, groups = kThreads / L;
+  const int g = threadIdx.x / L, l = threadIdx.x % L;
   double pq = 0.0;
-  for (int row = blockIdx.x * groups_per_block + g; row < n; row += gridDim.x * groups_per_block) {
-    const int64_t b = rowptr[row], e = rowptr[row + 1];
-    ACC s = 0;
-    for (int64_t k = b + l; k < e; k += LANES) s += (ACC)val[k] * (ACC)p[colind[k]];
-#pragma unroll
-    for (int off = LANES / 2; off >= 1; off >>= 1) s += __shfl_xor(s, off, LANES);
+  for (int row = blockIdx.x * groups + g; row < n; row += gridDim.x * groups) {
+    const int64_t b = rowptr[row];
+    const int cnt = (int)(rowptr[row + 1] - b);
+    ACC s = group_sum<L>(row_dot<L, ACC>(l, cnt, val + b, SHAPED ? cols + start[row] : cols + b,
+                                         SHAPED ? p + row : p));
     if (!std::is_same<VV, V>::value) s *= scale;
     if (l == 0) {
       q[row] = (V)s;
@@ -67,44 +74,36 @@ __global__ __launch_bounds__(kThreads) void k_spmv_dot(
 
 // SpMV for 3-component systems whose DOFs are free or fixed per node: the
 // three rows of a node share one column pattern made of node triples, so the
-// gather reads one node index (bcol) per 9 values.  One wave per node; the
+// gather reads one node index (bcol) per 9 values.  16 lanes per node; the
 // CSR values are read in place.  Blocks are mapped to the 8 XCDs in
 // contiguous node ranges so each XCD's L2 holds its slice of p.
-template <typename V, typename ACC, bool DOT, bool SKIP = DOT, typename VV = V>
+// SHAPED: node columns from the row shapes (start per node, table `cols`).
+// Bound by the reading of the values.  Elasticity 64^3 p = 2 FP64 (2.4 GB):
+// 524 us with one wave per node and column indices, 494 with row shapes, 427
+// (5.7 TB/s) with 16 lanes and four neighbours ahead per lane; 439 with 8
+// lanes, 455 with 32 and two ahead.
+template <typename V, typename ACC, bool DOT, bool SKIP = DOT, typename VV = V,
+          bool SHAPED = false>
 __global__ __launch_bounds__(kThreads) void k_spmv_node3(
-    int nnode, const int64_t* __restrict__ rowptr, const int32_t* __restrict__ bcol,
-    const VV* __restrict__ val, const V* __restrict__ p, V* __restrict__ q,
-    double* __restrict__ part_pq, const double* __restrict__ scal, ACC scale)
+    int nnode, const int64_t* __restrict__ rowptr, const int32_t* __restrict__ start,
+    const int32_t* __restrict__ cols, const VV* __restrict__ val, const V* __restrict__ p,
+    V* __restrict__ q, double* __restrict__ part_pq, const double* __restrict__ scal, ACC scale)
 {
   if (SKIP && scal[S_DONE] != 0.0) return;
   __shared__ double sh[kThreads / 64];
-  constexpr int WPB = kThreads / 64;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  constexpr int L = 16, GPB = kThreads / L;
+  const int g = threadIdx.x / L, lane = threadIdx.x % L;
   const int nxcd = 8;
   const int xcd = blockIdx.x % nxcd, bl = blockIdx.x / nxcd, nbl = gridDim.x / nxcd;
   const int lo = (int)((int64_t)nnode * xcd / nxcd), hi = (int)((int64_t)nnode * (xcd + 1) / nxcd);
   double pq = 0.0;
-  for (int nd = lo + bl * WPB + wave; nd < hi; nd += nbl * WPB) {
+  for (int nd = lo + bl * GPB + g; nd < hi; nd += nbl * GPB) {
     const int64_t r0 = rowptr[3 * nd];
     const int cnt = (int)((rowptr[3 * nd + 1] - r0) / 3);
-    const int64_t nb = r0 / 9;
-    const VV* v0 = val + r0;
-    const VV* v1 = v0 + 3 * cnt;
-    const VV* v2 = v1 + 3 * cnt;
-    ACC s0 = 0, s1 = 0, s2 = 0;
-    for (int k = lane; k < cnt; k += 64) {
-      const int64_t c = 3 * (int64_t)bcol[nb + k];
-      const ACC x0 = (ACC)p[c], x1 = (ACC)p[c + 1], x2 = (ACC)p[c + 2];
-      s0 += (ACC)v0[3 * k] * x0 + (ACC)v0[3 * k + 1] * x1 + (ACC)v0[3 * k + 2] * x2;
-      s1 += (ACC)v1[3 * k] * x0 + (ACC)v1[3 * k + 1] * x1 + (ACC)v1[3 * k + 2] * x2;
-      s2 += (ACC)v2[3 * k] * x0 + (ACC)v2[3 * k + 1] * x1 + (ACC)v2[3 * k + 2] * x2;
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-      s0 += __shfl_xor(s0, off, 64);
-      s1 += __shfl_xor(s1, off, 64);
-      s2 += __shfl_xor(s2, off, 64);
-    }
+    ACC t[3];
+    node_dots<L>(lane, cnt, val + r0, SHAPED ? cols + start[nd] : cols + r0 / 9,
+                     SHAPED ? p + 3 * (int64_t)nd : p, t);
+    ACC s0 = group_sum<L>(t[0]), s1 = group_sum<L>(t[1]), s2 = group_sum<L>(t[2]);
     if (!std::is_same<VV, V>::value) {
       s0 *= scale;
       s1 *= scale;
@@ -160,11 +159,11 @@ __device__ inline float hi_half(uint32_t w) { return __half2float(__ushort_as_ha
 // q = scale * (K16 p) with the node-block FP16 values (k_demote16_node3), FP32
 // sums: the fine-level smoother's SpMV.  Same wave-per-node and XCD mapping
 // as k_spmv_node3.
-template <bool SKIP>
+template <bool SKIP, bool SHAPED>
 __global__ __launch_bounds__(kThreads) void k_spmv_node3_h(
-    int nnode, const int64_t* __restrict__ rowptr, const int32_t* __restrict__ bcol,
-    const uint2* __restrict__ val, const float* __restrict__ p, float* __restrict__ q,
-    const double* __restrict__ scal, float scale)
+    int nnode, const int64_t* __restrict__ rowptr, const int32_t* __restrict__ start,
+    const int32_t* __restrict__ bcol, const uint2* __restrict__ val, const float* __restrict__ p,
+    float* __restrict__ q, const double* __restrict__ scal, float scale)
 {
   if (SKIP && scal[S_DONE] != 0.0) return;
   constexpr int WPB = kThreads / 64;
@@ -176,11 +175,13 @@ __global__ __launch_bounds__(kThreads) void k_spmv_node3_h(
     const int64_t r0 = rowptr[3 * nd];
     const int cnt = (int)((rowptr[3 * nd + 1] - r0) / 3);
     const int64_t nb = r0 / 9;
+    const int32_t* __restrict__ bc = SHAPED ? bcol + start[nd] : bcol + nb;
+    const float* __restrict__ pb = SHAPED ? p + 3 * (int64_t)nd : p;
     const uint2* vb = val + nb * 3;
     float s0 = 0.f, s1 = 0.f, s2 = 0.f;
     for (int k = lane; k < cnt; k += 64) {
-      const int64_t c = 3 * (int64_t)bcol[nb + k];
-      const float x0 = p[c], x1 = p[c + 1], x2 = p[c + 2];
+      const int64_t c = 3 * (int64_t)bc[k];
+      const float x0 = pb[c], x1 = pb[c + 1], x2 = pb[c + 2];
       const uint2 w0 = vb[3 * k], w1 = vb[3 * k + 1], w2 = vb[3 * k + 2];
       s0 += lo_half(w0.x) * x0 + hi_half(w0.x) * x1 + lo_half(w0.y) * x2;
       s1 += lo_half(w1.x) * x0 + hi_half(w1.x) * x1 + lo_half(w1.y) * x2;
@@ -355,36 +356,25 @@ __global__ void k_demote_scaled(int n, const double* __restrict__ r, float* __re
 }
 
 // ---------------------------------------------------------------------------
-static int lanes_for(const Context& c)
-{
-  const double avg = c.neq > 0 ? (double)c.nnz / c.neq : 0.0;
-  if (avg > 96) return 64;
-  if (avg > 40) return 32;
-  return 16;
-}
-
 template <typename V, typename ACC, bool DOT, bool SKIP = DOT, typename VV = V>
 static void launch_spmv(Context& c, const VV* val, const V* p, V* q, ACC scale = ACC(1),
                         hipStream_t st = nullptr)
 {
-  const int L = lanes_for(c);
-  SolverWork& w = c.w;
-  const int grid = kGrid;
+  const SolverWork& w = c.w;
+  const RowShapes& sh = c.shapes;
   if (!st) st = c.stream;
-  if (c.d_bcol) {
-    k_spmv_node3<V, ACC, DOT, SKIP, VV><<<grid, kThreads, 0, st>>>(
-        c.neq / 3, c.d_rowptr, c.d_bcol, val, p, q, w.partial, w.scal, scale);
-    return;
-  }
-  if (L == 64)
-    k_spmv_dot<V, ACC, 64, DOT, SKIP, VV><<<grid, kThreads, 0, st>>>(
-        c.neq, c.d_rowptr, c.d_colind, val, p, q, w.partial, w.scal, scale);
-  else if (L == 32)
-    k_spmv_dot<V, ACC, 32, DOT, SKIP, VV><<<grid, kThreads, 0, st>>>(
-        c.neq, c.d_rowptr, c.d_colind, val, p, q, w.partial, w.scal, scale);
+  auto run = [&](auto kernel, int n, const int32_t* start, const int32_t* cols) {
+    kernel<<<kGrid, kThreads, 0, st>>>(n, c.d_rowptr, start, cols, val, p, q, w.partial, w.scal,
+                                       scale);
+  };
+  if (c.d_bcol && sh.start)
+    run(k_spmv_node3<V, ACC, DOT, SKIP, VV, true>, c.neq / 3, sh.start, sh.table);
+  else if (c.d_bcol)
+    run(k_spmv_node3<V, ACC, DOT, SKIP, VV>, c.neq / 3, nullptr, c.d_bcol);
+  else if (sh.start)
+    run(k_spmv_dot<V, ACC, DOT, SKIP, VV, true>, c.neq, sh.start, sh.table);
   else
-    k_spmv_dot<V, ACC, 16, DOT, SKIP, VV><<<grid, kThreads, 0, st>>>(
-        c.neq, c.d_rowptr, c.d_colind, val, p, q, w.partial, w.scal, scale);
+    run(k_spmv_dot<V, ACC, DOT, SKIP, VV>, c.neq, nullptr, c.d_colind);
 }
 
 // FP32 SpMV for the multigrid smoother on the finest level.
@@ -414,12 +404,16 @@ void launch_spmv16_node3(Context& c, const uint2* val, float scale, const float*
                          bool skip_done, hipStream_t st)
 {
   if (!st) st = c.stream;
-  if (skip_done)
-    k_spmv_node3_h<true><<<kGrid, kThreads, 0, st>>>(c.neq / 3, c.d_rowptr, c.d_bcol, val, p, q,
-                                                      c.w.scal, scale);
+  const RowShapes& sh = c.shapes;
+  auto run = [&](auto kernel, const int32_t* start, const int32_t* cols) {
+    kernel<<<kGrid, kThreads, 0, st>>>(c.neq / 3, c.d_rowptr, start, cols, val, p, q, c.w.scal, scale);
+  };
+  if (sh.start)
+    skip_done ? run(k_spmv_node3_h<true, true>, sh.start, sh.table)
+              : run(k_spmv_node3_h<false, true>, sh.start, sh.table);
   else
-    k_spmv_node3_h<false><<<kGrid, kThreads, 0, st>>>(c.neq / 3, c.d_rowptr, c.d_bcol, val, p, q,
-                                                       c.w.scal, scale);
+    skip_done ? run(k_spmv_node3_h<true, false>, nullptr, c.d_bcol)
+              : run(k_spmv_node3_h<false, false>, nullptr, c.d_bcol);
 }
 
 int spmv_device(Context& c, const double* d_x, double* d_y)
@@ -477,6 +471,10 @@ int solver_setup(Context& c)
     k_build_bcol<<<c.neq / 3, 128, 0, c.stream>>>(c.neq / 3, c.d_rowptr, c.d_colind, c.d_bcol);
     IFEM_HIP(hipGetLastError());
   }
+  int rc = build_row_shapes(c.stream, uniform ? c.neq / 3 : c.neq, c.d_rowptr,
+                            uniform ? c.d_bcol : c.d_colind, uniform,
+                            uniform ? c.nnz / 9 : c.nnz, c.shapes);
+  if (rc) return rc;
   w.nblocks = kGrid;
   IFEM_HIP(hipStreamSynchronize(c.stream));
   return IFEM_GPU_OK;

@@ -400,8 +400,8 @@ int ifem_gpu_batch_init(ifem_gpu_ctx* ctx, int* neq, int64_t* nnz);
  * first: IFEM_GPU_FP64 writes K and b, IFEM_GPU_FP32 the FP32 copy of K. */
 int ifem_gpu_batch_assemble(ifem_gpu_ctx* ctx, int precision);
 /* Tunes, for each degree present (nen = (p+1)^3 element nodes), the element
- * chunk of the assembly (full or half) and the SpMV lanes per row
- * (16/32/64) by timing the batch, then re-assembles with the choice.
+ * chunk of the assembly (full or half) and the row entries per SpMV step
+ * (16/32/64, two per lane) by timing the batch, then re-assembles with the choice.
  * table (may be NULL) receives 4 x {half, lanes} indexed by p. */
 int ifem_gpu_batch_autotune(ifem_gpu_ctx* ctx, int precision, int* table);
 /* Solves every patch to max(rtol*||b_q||, atol) on its true FP64 residual;
