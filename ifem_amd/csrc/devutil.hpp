@@ -17,7 +17,7 @@ enum Scal {
   S_NSCAL
 };
 
-template <typename A>
+template <typename A, int T = kThreads>
 __device__ inline A block_sum(A v, A* sh)
 {
   // fixed-shape reduction: wave butterflies, then wave totals in order;
@@ -28,16 +28,17 @@ __device__ inline A block_sum(A v, A* sh)
   if (lane == 0) sh[wave] = v;
   __syncthreads();
   A s = 0;
-  for (int w = 0; w < kThreads / 64; w++) s += sh[w];
+  for (int w = 0; w < T / 64; w++) s += sh[w];
   return s;
 }
 
 // Sum of nparts partials in index order, computed by the whole block.
+template <int T = kThreads>
 __device__ inline double sum_parts(const double* __restrict__ part, int nparts, double* sh)
 {
   double s = 0.0;
-  for (int i = threadIdx.x; i < nparts; i += kThreads) s += part[i];
-  return block_sum<double>(s, sh);
+  for (int i = threadIdx.x; i < nparts; i += T) s += part[i];
+  return block_sum<double, T>(s, sh);
 }
 
 // Jacobi: inverse of the diagonal of A (CSR rows sorted: binary search).

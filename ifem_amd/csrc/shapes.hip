@@ -37,6 +37,7 @@ struct ShapeRows {
   }
 };
 
+// Finaliser of the splitmix64 generator (Steele, Lea and Flood, 2014).
 __device__ inline uint64_t mix64(uint64_t z)
 {
   z += 0x9E3779B97F4A7C15ull;
@@ -124,20 +125,27 @@ __global__ void k_shape_check(ShapeRows R, int n, int total, const int32_t* __re
 __global__ void k_shape_clear(int* bad) { *bad = 0; }
 
 static int build(hipStream_t s, int n, const ShapeRows& R, int64_t entries, RowShapes& out,
-                 void* (&tmp)[8])
+                 void* (&tmp)[4])
 {
   uint64_t *key = nullptr, *skey = nullptr;
   int *row = nullptr, *srow = nullptr, *head = nullptr, *len = nullptr;
   int64_t* incl = nullptr;
-  IFEM_HIP(hipMalloc(&tmp[0], sizeof(uint64_t) * 2 * (size_t)n));
+  // without memory for the search the products keep the column indices
+  auto alloc = [](void** p, size_t bytes) {
+    if (hipMalloc(p, bytes) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+  };
+  if (!alloc(&tmp[0], sizeof(uint64_t) * 2 * (size_t)n) ||
+      !alloc(&tmp[1], sizeof(int) * 4 * (size_t)n) ||
+      !alloc(&tmp[2], sizeof(int64_t) * ((size_t)n + 1)))
+    return IFEM_GPU_OK;
   key = static_cast<uint64_t*>(tmp[0]);
   skey = key + n;
-  IFEM_HIP(hipMalloc(&tmp[1], sizeof(int) * 4 * (size_t)n));
   row = static_cast<int*>(tmp[1]);
   srow = row + n;
   head = srow + n;
   len = head + n;
-  IFEM_HIP(hipMalloc(&tmp[2], sizeof(int64_t) * ((size_t)n + 1)));
   incl = static_cast<int64_t*>(tmp[2]);
   int* bad = reinterpret_cast<int*>(incl + n);
   const unsigned nb = (unsigned)((n + 255) / 256), nwv = (unsigned)((n + 3) / 4 < 8192 ? (n + 3) / 4 : 8192);
@@ -145,7 +153,7 @@ static int build(hipStream_t s, int n, const ShapeRows& R, int64_t entries, RowS
   size_t tb = 0, tb2 = 0;
   IFEM_HIP(rocprim::radix_sort_pairs(nullptr, tb, key, skey, row, srow, (size_t)n, 0, 64, s));
   IFEM_HIP(rocprim::inclusive_scan(nullptr, tb2, len, incl, (size_t)n, rocprim::plus<int64_t>(), s));
-  IFEM_HIP(hipMalloc(&tmp[3], tb > tb2 ? tb : tb2));
+  if (!alloc(&tmp[3], tb > tb2 ? tb : tb2)) return IFEM_GPU_OK;
   IFEM_HIP(rocprim::radix_sort_pairs(tmp[3], tb, key, skey, row, srow, (size_t)n, 0, 64, s));
   k_shape_heads<<<nb, 256, 0, s>>>(R, n, skey, srow, head, len);
   IFEM_HIP(rocprim::inclusive_scan(tmp[3], tb2, len, incl, (size_t)n, rocprim::plus<int64_t>(), s));
@@ -153,8 +161,11 @@ static int build(hipStream_t s, int n, const ShapeRows& R, int64_t entries, RowS
   IFEM_HIP(hipMemcpyAsync(&total, incl + n - 1, sizeof(int64_t), hipMemcpyDeviceToHost, s));
   IFEM_HIP(hipStreamSynchronize(s));
   if (total > entries / 8 || total > INT32_MAX) return IFEM_GPU_OK; // mostly distinct
-  IFEM_HIP(hipMalloc(&out.start, sizeof(int32_t) * (size_t)n));
-  IFEM_HIP(hipMalloc(&out.table, sizeof(int32_t) * (size_t)(total > 0 ? total : 1)));
+  if (!alloc((void**)&out.start, sizeof(int32_t) * (size_t)n) ||
+      !alloc((void**)&out.table, sizeof(int32_t) * (size_t)(total > 0 ? total : 1))) {
+    out.release();
+    return IFEM_GPU_OK;
+  }
   k_shape_assign<<<nb, 256, 0, s>>>(n, srow, incl, R, out.start);
   k_shape_table<<<nwv, 256, 0, s>>>(R, n, srow, head, out.start, out.table);
   k_shape_clear<<<1, 1, 0, s>>>(bad);
@@ -172,7 +183,7 @@ int build_row_shapes(hipStream_t s, int n, const int64_t* rowptr, const int32_t*
 {
   out.release();
   if (n <= 0 || entries <= 0) return IFEM_GPU_OK;
-  void* tmp[8] = {};
+  void* tmp[4] = {};
   const int rc = build(s, n, ShapeRows{rowptr, cols, nodal ? 1 : 0}, entries, out, tmp);
   for (void* t : tmp) hipFree(t);
   if (rc) out.release();

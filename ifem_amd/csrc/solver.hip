@@ -6,14 +6,14 @@
 // src/LinAlg/ISTLMatrix.C:169-196), with the LinSolParams convergence
 // contract (rtol, atol, maxits; src/LinAlg/LinSolParams.C:68-77).
 //
-// One iteration is three launches on a fixed grid:
+// One iteration is three launches:
 //   k_spmv_dot : q = A p, per-block partials of <p,q>
 //   k_update   : alpha = rz / sum(partials <p,q>); x += alpha p,
 //                r -= alpha q, z = D^-1 r; per-block partials <r,z>, <r,r>
 //   k_pupdate  : beta = sum(<r,z>) / rz; p = z + beta p; block 0 records the
 //                scalars (rz, rr, iteration count, convergence flag)
-// Every block that needs a global sum reduces the 2048 per-block partials
-// itself, in index order, so all blocks agree bitwise and no grid-wide fence
+// Every block that needs a global sum reduces the per-block partials itself,
+// in a fixed order, so all blocks agree bitwise and no grid-wide fence
 // or atomic is needed (a device-scope fence per block forces L2 write-backs
 // across the XCDs).  Scalars stay on the device; the host reads them every
 // check_every iterations.  Results are bitwise reproducible run to run.
@@ -34,6 +34,9 @@
 
 namespace ifem {
 
+constexpr int kRowLanes = 8, kNodeLanes = 16; // lanes of the products per row, per node
+constexpr int kUpd = 512;                     // threads of the update kernels
+
 // ---------------------------------------------------------------------------
 // SpMV q = A p (CSR), 8 lanes per row; with DOT, per-block partial <p,q>.
 // SKIP: return at once when scal[S_DONE] is set (work queued past convergence).
@@ -53,7 +56,7 @@ __global__ __launch_bounds__(kThreads) void k_spmv_dot(
 {
   if (SKIP && scal[S_DONE] != 0.0) return;
   __shared__ double sh[kThreads / 64];
-  constexpr int L = 8, groups = kThreads / L;
+  constexpr int L = kRowLanes, groups = kThreads / L;
   const int g = threadIdx.x / L, l = threadIdx.x % L;
   double pq = 0.0;
   for (int row = blockIdx.x * groups + g; row < n; row += gridDim.x * groups) {
@@ -91,7 +94,7 @@ __global__ __launch_bounds__(kThreads) void k_spmv_node3(
 {
   if (SKIP && scal[S_DONE] != 0.0) return;
   __shared__ double sh[kThreads / 64];
-  constexpr int L = 16, GPB = kThreads / L;
+  constexpr int L = kNodeLanes, GPB = kThreads / L;
   const int g = threadIdx.x / L, lane = threadIdx.x % L;
   const int nxcd = 8;
   const int xcd = blockIdx.x % nxcd, bl = blockIdx.x / nxcd, nbl = gridDim.x / nxcd;
@@ -211,36 +214,48 @@ __global__ void k_build_bcol(int nnode, const int64_t* __restrict__ rowptr,
   for (int k = threadIdx.x; k < cnt; k += blockDim.x) bcol[r0 / 9 + k] = colind[r0 + 3 * k] / 3;
 }
 
+// Bound by the launch and by every block's sum of the product's partials.
+// One block of 512 per CU has few partials to write and to read again, and its
+// first loads are under way while it adds up: 2048 blocks of 256 (with 2048
+// partials of the product) took 7 to 8 us for 0.1 to 0.2 M unknowns.  Jacobi-
+// PCG of diffusion 48^3: 5.42 -> 4.67 ms; 8^3: 1.32 -> 0.90 ms; 1024 threads
+// or 512 and 1024 blocks of 256 gain less.
 template <typename V>
-__global__ __launch_bounds__(kThreads) void k_update(int n, V* __restrict__ x, V* __restrict__ r,
-                                                     V* __restrict__ z, const V* __restrict__ p,
-                                                     const V* __restrict__ q,
-                                                     const V* __restrict__ dinv,
-                                                     const double* __restrict__ part_pq,
-                                                     double* __restrict__ part_rz,
-                                                     double* __restrict__ part_rr,
-                                                     double* __restrict__ scal, int parity)
+__global__ __launch_bounds__(kUpd) void k_update(int n, V* __restrict__ x, V* __restrict__ r,
+                                                 V* __restrict__ z, const V* __restrict__ p,
+                                                 const V* __restrict__ q,
+                                                 const V* __restrict__ dinv,
+                                                 const double* __restrict__ part_pq, int npq,
+                                                 double* __restrict__ part_rz,
+                                                 double* __restrict__ part_rr,
+                                                 double* __restrict__ scal, int parity)
 {
   if (scal[S_DONE] != 0.0) return;
-  __shared__ double sh[kThreads / 64];
-  const double pq = sum_parts(part_pq, gridDim.x, sh);
+  __shared__ double sh[kUpd / 64];
+  // the first entry's loads go out before the partials are summed
+  int i = blockIdx.x * kUpd + threadIdx.x;
+  V xi = 0, pi = 0, ri = 0, qi = 0, di = 0;
+  if (i < n) xi = x[i], pi = p[i], ri = r[i], qi = q[i], di = dinv[i];
+  const double pq = sum_parts<kUpd>(part_pq, npq, sh);
   double a = 0.0;
   if (pq != 0.0 && __builtin_isfinite(pq)) a = scal[S_RZ + parity] / pq;
   else if (blockIdx.x == 0 && threadIdx.x == 0) scal[S_DONE] = 2.0; // breakdown
   const V alpha = (V)a;
   double rz = 0.0, rr = 0.0;
-  for (int i = blockIdx.x * kThreads + threadIdx.x; i < n; i += gridDim.x * kThreads) {
-    const V xi = x[i] + alpha * p[i];
-    const V ri = r[i] - alpha * q[i];
-    const V zi = dinv[i] * ri;
+  while (i < n) {
+    xi += alpha * pi;
+    ri -= alpha * qi;
+    const V zi = di * ri;
     x[i] = xi;
     r[i] = ri;
     z[i] = zi;
     rz += (double)(ri * zi);
     rr += (double)(ri * ri);
+    i += gridDim.x * kUpd;
+    if (i < n) xi = x[i], pi = p[i], ri = r[i], qi = q[i], di = dinv[i];
   }
-  const double brz = block_sum<double>(rz, sh);
-  const double brr = block_sum<double>(rr, sh);
+  const double brz = block_sum<double, kUpd>(rz, sh);
+  const double brr = block_sum<double, kUpd>(rr, sh);
   if (threadIdx.x == 0) {
     part_rz[blockIdx.x] = brz;
     part_rr[blockIdx.x] = brr;
@@ -248,16 +263,19 @@ __global__ __launch_bounds__(kThreads) void k_update(int n, V* __restrict__ x, V
 }
 
 template <typename V>
-__global__ __launch_bounds__(kThreads) void k_pupdate(int n, V* __restrict__ p,
-                                                      const V* __restrict__ z,
-                                                      const double* __restrict__ part_rz,
-                                                      const double* __restrict__ part_rr,
-                                                      double* __restrict__ scal, int parity)
+__global__ __launch_bounds__(kUpd) void k_pupdate(int n, V* __restrict__ p,
+                                                  const V* __restrict__ z,
+                                                  const double* __restrict__ part_rz,
+                                                  const double* __restrict__ part_rr,
+                                                  double* __restrict__ scal, int parity)
 {
   if (scal[S_DONE] != 0.0) return;
-  __shared__ double sh[kThreads / 64];
-  const double rzn = sum_parts(part_rz, gridDim.x, sh);
-  const double rr = sum_parts(part_rr, gridDim.x, sh);
+  __shared__ double sh[kUpd / 64];
+  int i = blockIdx.x * kUpd + threadIdx.x;
+  V zi = 0, pi = 0;
+  if (i < n) zi = z[i], pi = p[i];
+  const double rzn = sum_parts<kUpd>(part_rz, gridDim.x, sh);
+  const double rr = sum_parts<kUpd>(part_rr, gridDim.x, sh);
   const double rzo = scal[S_RZ + parity];
   const bool conv = !(rr > scal[S_TOL2]); // converged (or NaN)
   if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -269,8 +287,11 @@ __global__ __launch_bounds__(kThreads) void k_pupdate(int n, V* __restrict__ p,
   }
   if (conv) return;
   const V beta = (V)(rzo != 0.0 ? rzn / rzo : 0.0);
-  for (int i = blockIdx.x * kThreads + threadIdx.x; i < n; i += gridDim.x * kThreads)
-    p[i] = z[i] + beta * p[i];
+  while (i < n) {
+    p[i] = zi + beta * pi;
+    i += gridDim.x * kUpd;
+    if (i < n) zi = z[i], pi = p[i];
+  }
 }
 
 // CG start from residual r (already in place): z = D^-1 r, p = z, partials.
@@ -356,6 +377,27 @@ __global__ void k_demote_scaled(int n, const double* __restrict__ r, float* __re
 }
 
 // ---------------------------------------------------------------------------
+// Blocks of a product (a multiple of the 8 XCDs): one pass over the rows where
+// that takes few, else 4 per CU, 8 for FP64 node triples.  4 leave the CUs
+// evenly loaded and half the partials to add up: mixed elasticity step 40^3
+// 49.0 against 50.7 ms, Jacobi-PCG of diffusion 48^3 4.54 against 4.67 ms;
+// FP64 triples fit 4 blocks at a time and read faster when more are queued
+// (elasticity 64^3 400 against 405 ms a solve).
+template <typename V>
+static int spmv_grid(const Context& c)
+{
+  const int rows = c.d_bcol ? c.neq / 3 : c.neq, per = kThreads / (c.d_bcol ? kNodeLanes : kRowLanes);
+  const int need = (rows + per - 1) / per, cap = c.d_bcol && sizeof(V) == 8 ? kGrid : kGrid / 2;
+  return need < cap ? (need + 7) / 8 * 8 : cap;
+}
+
+// Blocks of the update kernels: one per CU, see k_update.
+static int upd_grid(int n)
+{
+  const int need = (n + kUpd - 1) / kUpd;
+  return need < 256 ? need : 256;
+}
+
 template <typename V, typename ACC, bool DOT, bool SKIP = DOT, typename VV = V>
 static void launch_spmv(Context& c, const VV* val, const V* p, V* q, ACC scale = ACC(1),
                         hipStream_t st = nullptr)
@@ -363,8 +405,9 @@ static void launch_spmv(Context& c, const VV* val, const V* p, V* q, ACC scale =
   const SolverWork& w = c.w;
   const RowShapes& sh = c.shapes;
   if (!st) st = c.stream;
+  const int grid = spmv_grid<V>(c);
   auto run = [&](auto kernel, int n, const int32_t* start, const int32_t* cols) {
-    kernel<<<kGrid, kThreads, 0, st>>>(n, c.d_rowptr, start, cols, val, p, q, w.partial, w.scal,
+    kernel<<<grid, kThreads, 0, st>>>(n, c.d_rowptr, start, cols, val, p, q, w.partial, w.scal,
                                        scale);
   };
   if (c.d_bcol && sh.start)
@@ -517,14 +560,15 @@ static int pcg_run(Context& c, const V* val, V* x, V* r, V* z, V* p, V* q, const
   k_start<V><<<kGrid, kThreads, 0, c.stream>>>(n, r, z, p, dinv, part_rz, part_rr);
   k_start_check<<<1, kThreads, 0, c.stream>>>(part_rz, part_rr, kGrid, w.scal);
   IFEM_HIP(hipGetLastError());
+  const int npq = spmv_grid<V>(c), gupd = upd_grid(n);
   int launched = 0;
   while (true) {
     for (int k = 0; k < check_every; k++) {
       const int parity = (launched + k) & 1;
       launch_spmv<V, ACC, true>(c, val, p, q);
-      k_update<V><<<kGrid, kThreads, 0, c.stream>>>(n, x, r, z, p, q, dinv, part_pq, part_rz,
-                                                    part_rr, w.scal, parity);
-      k_pupdate<V><<<kGrid, kThreads, 0, c.stream>>>(n, p, z, part_rz, part_rr, w.scal, parity);
+      k_update<V><<<gupd, kUpd, 0, c.stream>>>(n, x, r, z, p, q, dinv, part_pq, npq, part_rz,
+                                               part_rr, w.scal, parity);
+      k_pupdate<V><<<gupd, kUpd, 0, c.stream>>>(n, p, z, part_rz, part_rr, w.scal, parity);
     }
     IFEM_HIP(hipGetLastError());
     launched += check_every;
@@ -548,13 +592,13 @@ __global__ __launch_bounds__(kThreads) void k_update_f(int n, V* __restrict__ x,
                                                        V* __restrict__ rold,
                                                        const V* __restrict__ p,
                                                        const V* __restrict__ q,
-                                                       const double* __restrict__ part_pq,
+                                                       const double* __restrict__ part_pq, int npq,
                                                        double* __restrict__ part_rr,
                                                        double* __restrict__ scal, int parity)
 {
   if (scal[S_DONE] != 0.0) return;
   __shared__ double sh[kThreads / 64];
-  const double pq = sum_parts(part_pq, gridDim.x, sh);
+  const double pq = sum_parts(part_pq, npq, sh);
   double a = 0.0;
   if (pq != 0.0 && __builtin_isfinite(pq)) a = scal[S_RZ + parity] / pq;
   else if (blockIdx.x == 0 && threadIdx.x == 0) scal[S_DONE] = 2.0;
@@ -903,12 +947,13 @@ static int fcg_run(Context& c, int kind, const V* val, V* x, V* r, V* z, V* zn, 
     k_copy<V><<<(n + 255) / 256, 256, 0, c.stream>>>(n, z, p);
   }
   IFEM_HIP(hipGetLastError());
+  const int npq = spmv_grid<V>(c);
   int launched = 0;
   while (true) {
     for (int k = 0; k < check_every; k++) {
       const int parity = (launched + k) & 1;
       launch_spmv<V, ACC, true>(c, val, p, q);
-      k_update_f<V><<<kGrid, kThreads, 0, c.stream>>>(n, x, r, rold, p, q, part_pq, part_rr,
+      k_update_f<V><<<kGrid, kThreads, 0, c.stream>>>(n, x, r, rold, p, q, part_pq, npq, part_rr,
                                                       w.scal, parity);
       if (learned) {
         rc = apply_learned<V>(c, mg_base, r, rold, dinv, z, zn, part_rr, part4);
