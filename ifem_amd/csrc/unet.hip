@@ -45,6 +45,7 @@ namespace ifem {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+typedef __attribute__((__vector_size__(4 * sizeof(short)))) short i16x4;
 
 __device__ inline float bf2f(uint32_t h) { return __uint_as_float(h << 16); }
 // round to nearest even
@@ -75,34 +76,41 @@ __device__ inline uint4 pack8(const float* f)
 }
 
 // 8 channels [c, c+8) of a convolution input at voxel (z, y, x) of sample n
-// (output resolution D x H x W); zero outside the volume.
+// (output resolution D x H x W); zero outside the volume.  POOLED: in0 may be
+// at twice the resolution (mode 2).  One load with a selected source: 64-bit
+// index chains in a branch per source were most of the convolutions' vector
+// instructions.
+template <bool POOLED>
 __device__ inline uint4 load8(const ConvIn& in, int n, int D, int H, int W, int z, int y, int x,
                               int c)
 {
   uint4 r = make_uint4(0u, 0u, 0u, 0u);
-  if (z < 0 || z >= D || y < 0 || y >= H || x < 0 || x >= W) return r;
-  if (c >= in.c0p)
-    return *(const uint4*)(in.in1 + ((((int64_t)n * D + z) * H + y) * W + x) * in.c1p +
-                           (c - in.c0p));
-  if (in.mode0 == 0)
-    return *(const uint4*)(in.in0 + ((((int64_t)n * D + z) * H + y) * W + x) * in.c0p + c);
-  if (in.mode0 == 1) {
-    const int d = D >> 1, h = H >> 1, w = W >> 1;
-    return *(const uint4*)(in.in0 + ((((int64_t)n * d + (z >> 1)) * h + (y >> 1)) * w + (x >> 1)) *
-                                        in.c0p + c);
+  if ((unsigned)z >= (unsigned)D || (unsigned)y >= (unsigned)H || (unsigned)x >= (unsigned)W)
+    return r;
+  const bool second = c >= in.c0p;
+  if (POOLED && in.mode0 == 2 && !second) {
+    const int D2 = 2 * D, H2 = 2 * H, W2 = 2 * W;
+    float s[8] = {0, 0, 0, 0, 0, 0, 0, 0}, f[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      const int zz = 2 * z + (q >> 2), yy = 2 * y + ((q >> 1) & 1), xx = 2 * x + (q & 1);
+      unpack8(*(const uint4*)(in.in0 + ((((int64_t)n * D2 + zz) * H2 + yy) * W2 + xx) * in.c0p + c),
+              f);
+#pragma unroll
+      for (int i = 0; i < 8; i++) s[i] += f[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) s[i] *= 0.125f;
+    return pack8(s);
   }
-  const int D2 = 2 * D, H2 = 2 * H, W2 = 2 * W;
-  float s[8] = {0, 0, 0, 0, 0, 0, 0, 0}, f[8];
-#pragma unroll
-  for (int q = 0; q < 8; q++) {
-    const int zz = 2 * z + (q >> 2), yy = 2 * y + ((q >> 1) & 1), xx = 2 * x + (q & 1);
-    unpack8(*(const uint4*)(in.in0 + ((((int64_t)n * D2 + zz) * H2 + yy) * W2 + xx) * in.c0p + c), f);
-#pragma unroll
-    for (int i = 0; i < 8; i++) s[i] += f[i];
-  }
-#pragma unroll
-  for (int i = 0; i < 8; i++) s[i] *= 0.125f;
-  return pack8(s);
+  const int sh = in.mode0 == 1 ? 1 : 0; // in0 at half the resolution
+  const int h0 = H >> sh, w0 = W >> sh;
+  const uint16_t* b0 = in.in0 + (int64_t)n * (D >> sh) * h0 * w0 * in.c0p;
+  const uint16_t* b1 = in.in1 + (int64_t)n * D * H * W * in.c1p;
+  const uint32_t v0 = ((uint32_t)(z >> sh) * h0 + (y >> sh)) * w0 + (x >> sh);
+  const uint32_t v1 = ((uint32_t)z * H + y) * W + x;
+  return *(const uint4*)((second ? b1 : b0) + (uint64_t)(second ? v1 : v0) * (second ? in.c1p : in.c0p) +
+                         (second ? c - in.c0p : c));
 }
 
 // ---------------------------------------------------------------------------
@@ -111,6 +119,7 @@ constexpr int BX = 16, BY = 4, BZ = 4;           // output brick
 constexpr int HXs = BX + 2, HYs = BY + 2, HZs = BZ + 2;
 constexpr int HVOX = HXs * HYs * HZs;             // 648 halo voxels
 constexpr int CCMAX = 32;                         // input channels per K chunk
+constexpr int kWhere = 4 * 27;                    // (step, lane group) pairs of a full chunk
 
 struct ConvArgs {
   ConvIn x;
@@ -131,13 +140,20 @@ __host__ __device__ inline int conv_bricks(int D, int H, int W)
   return ((W + BX - 1) / BX) * ((H + BY - 1) / BY) * ((D + BZ - 1) / BZ);
 }
 
-template <int NT>
-__global__ __launch_bounds__(256) void k_conv(ConvArgs a)
+// Bound by latency and by the vector instructions around the products: the
+// halo's loads go out together, the weights of PF steps while the steps before
+// them are multiplied, and where a lane's 8 contraction entries of a step lie
+// in the tile comes from a table (the divisions by the chunk's channel count
+// took half the instructions).  885k voxels, 12 channels: 43.5 -> 36.7 us
+// (steps unrolled with constant chunk sizes: 50, at half the waves).
+template <int NT, bool POOLED>
+__global__ __launch_bounds__(256, NT == 1 ? 5 : 1) void k_conv(ConvArgs a)
 {
   if (a.skip && *a.skip != 0.0) return;
   // halo tile of up to CCMAX input channels, sized by the launch to the
   // channels this convolution has (fewer channels: more blocks per CU)
   extern __shared__ uint4 tile[];
+  constexpr int PF = NT == 1 ? 4 : NT == 2 ? 2 : 1; // steps whose weights are requested at once
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int tb = blockIdx.z * NT; // first 16-channel output tile of this block
   const int row = lane & 15, grp = lane >> 4;
@@ -146,6 +162,7 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a)
   const int x0 = (b % nbx) * BX, y0 = ((b / nbx) % nby) * BY, z0 = (b / (nbx * nby)) * BZ;
   const int n = blockIdx.y;
   const int cin_p = a.x.c0p + a.x.c1p;
+  int* where = (int*)(tile + HVOX * (min(cin_p, CCMAX) / 8)); // behind the tile, kWhere entries
   f32x4 acc[4][NT];
 #pragma unroll
   for (int m = 0; m < 4; m++)
@@ -155,34 +172,60 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a)
   int kb_base = 0;
   for (int c_lo = 0; c_lo < cin_p; c_lo += CCMAX) {
     const int cc = min(CCMAX, cin_p - c_lo);
-    const int ng8 = cc >> 3;
-    __syncthreads();
-    for (int t = threadIdx.x; t < HVOX * ng8; t += 256) {
-      const int g8 = t % ng8, v = t / ng8;
-      const int hx = v % HXs, hy = (v / HXs) % HYs, hz = v / (HXs * HYs);
-      tile[t] = load8(a.x, n, a.D, a.H, a.W, z0 + hz - 1, y0 + hy - 1, x0 + hx - 1, c_lo + 8 * g8);
-    }
-    __syncthreads();
-    const int nkb = (27 * cc + 31) / 32;
-    for (int kb = 0; kb < nkb; kb++) {
-      const int kl = kb * 32 + grp * 8;
-      const int tap0 = kl / cc;
-      const int cl = kl - tap0 * cc;
-      const int tap = tap0 > 26 ? 26 : tap0; // padding of the last block: zero weights
-      const int dz = tap / 9, dy = (tap / 3) % 3, dx = tap % 3;
-      bf16x8 bw[NT];
+    const int ng8 = cc >> 3, nkb = (27 * cc + 31) / 32;
+    const uint16_t* wp = a.wp + (int64_t)(tb * 16 + row) * wrow + kb_base * 32 + grp * 8;
+    auto weights = [&](bf16x8 (&w)[PF][NT], int k0) {
 #pragma unroll
-      for (int t = 0; t < NT; t++)
-        bw[t] = __builtin_bit_cast(
-            bf16x8, *(const uint4*)(a.wp + (int64_t)((tb + t) * 16 + row) * wrow + (kb_base + kb) * 32 + grp * 8));
-#pragma unroll
-      for (int m = 0; m < 4; m++) {
-        const int hv = ((wave + dz) * HYs + (m + dy)) * HXs + (row + dx);
-        const bf16x8 av = __builtin_bit_cast(bf16x8, tile[hv * ng8 + (cl >> 3)]);
+      for (int k = 0; k < PF; k++)
 #pragma unroll
         for (int t = 0; t < NT; t++)
-          acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bw[t], acc[m][t], 0, 0, 0);
+          w[k][t] = __builtin_bit_cast(
+              bf16x8, *(const uint4*)(wp + t * 16 * wrow + 32 * min(k0 + k, nkb - 1)));
+    };
+    bf16x8 bw[PF][NT], bn[PF][NT];
+    weights(bw, 0);
+    __syncthreads();
+    if (threadIdx.x < 4 * nkb) { // tile entry of contraction index 8 threadIdx.x
+      const int kl = 8 * threadIdx.x, t0 = kl / cc, tap = t0 > 26 ? 26 : t0; // past 26: zero weights
+      where[threadIdx.x] =
+          (((tap / 9) * HYs + (tap / 3) % 3) * HXs + tap % 3) * ng8 + ((kl - t0 * cc) >> 3);
+    }
+    // HB entries per thread are requested before the first is stored
+    constexpr int HB = POOLED ? 1 : 6;
+    for (int t0 = threadIdx.x; t0 < HVOX * ng8; t0 += 256 * HB) {
+      uint4 h[HB];
+#pragma unroll
+      for (int i = 0; i < HB; i++) {
+        const int t = t0 + 256 * i, g8 = t % ng8, v = t / ng8;
+        const int hx = v % HXs, hy = (v / HXs) % HYs, hz = v / (HXs * HYs);
+        if (t < HVOX * ng8)
+          h[i] = load8<POOLED>(a.x, n, a.D, a.H, a.W, z0 + hz - 1, y0 + hy - 1, x0 + hx - 1,
+                               c_lo + 8 * g8);
       }
+#pragma unroll
+      for (int i = 0; i < HB; i++)
+        if (t0 + 256 * i < HVOX * ng8) tile[t0 + 256 * i] = h[i];
+    }
+    __syncthreads();
+    const uint4* tl = tile + (wave * HYs * HXs + row) * ng8;
+    for (int k0 = 0; k0 < nkb; k0 += PF) {
+      if (k0 + PF < nkb) weights(bn, k0 + PF);
+#pragma unroll
+      for (int k = 0; k < PF; k++) {
+        if (k0 + k >= nkb) break;
+        const uint4* tk = tl + where[4 * (k0 + k) + grp];
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+          const bf16x8 av = __builtin_bit_cast(bf16x8, tk[m * HXs * ng8]);
+#pragma unroll
+          for (int t = 0; t < NT; t++)
+            acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bw[k][t], acc[m][t], 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < PF; k++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) bw[k][t] = bn[k][t];
     }
     kb_base += nkb;
   }
@@ -243,11 +286,37 @@ struct WgradArgs {
   float* partb;      // [gridDim.x][MT*16] (blockIdx.y == 0)
 };
 
-template <int MT>
-__global__ __launch_bounds__(256) void k_wgrad(WgradArgs a)
+// Four consecutive voxels of channel (lane & 15) from a tile [voxel][channel]:
+// the 16 lanes of a group pass the addresses of 4 channels each (4 (lane & 3)
+// of voxel (lane >> 2) & 3) and get the 4 x 16 block transposed.
+__device__ inline i16x4 read_tr(const uint16_t* p)
 {
-  __shared__ __attribute__((aligned(16))) uint16_t gT[MT * 16][256];
-  __shared__ __attribute__((aligned(16))) uint16_t xT[3][16][HZs][HYs][BX];
+  typedef __attribute__((address_space(3))) i16x4 lds_t;
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_t*)p);
+}
+
+__device__ inline bf16x8 join(i16x4 lo, i16x4 hi)
+{
+  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+// Blocks walk the bricks; voxels are the contraction index, so both operands
+// are wanted with the voxels of one channel side by side while memory has the
+// channels of one voxel.  The tiles stay as they come (16-byte stores) and
+// the transposing LDS read turns them on the way to the matrix cores; a
+// brick's loads are under way while the one before is multiplied.  The bias
+// gradient is a 28th tap whose input is 1.  Bound by the LDS reads (16 per 8
+// matrix instructions at MT = 1) and the brick loads.  Tiles transposed by
+// 2-byte stores, one per x shift, and a bias sum by a few threads took 108 us
+// where this takes 48 (885k voxels, 12 channels; 42 with 3 blocks per CU, which
+// costs the wider layers as much).
+template <int MT, bool POOLED>
+__global__ __launch_bounds__(256, MT <= 2 ? 2 : 1) void k_wgrad(WgradArgs a)
+{
+  constexpr int GS = MT * 16;                      // channels per voxel of the gradient tile
+  constexpr int NG = MT * 2, NX = (HVOX * 2 + 255) / 256;
+  __shared__ __attribute__((aligned(16))) uint16_t gl[256 * GS];
+  __shared__ __attribute__((aligned(16))) uint16_t xl[HVOX * 16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int row = lane & 15, grp = lane >> 4;
   const int cig = blockIdx.y;
@@ -260,47 +329,41 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradArgs a)
   for (int m = 0; m < MT; m++)
 #pragma unroll
     for (int j = 0; j < 7; j++) acc[m][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float bsum = 0.f;
-  for (int64_t br = blockIdx.x; br < total; br += gridDim.x) {
+  uint4 gr[NG], xr[NX];
+  auto load = [&](int64_t br) {
     const int n = (int)(br / nbr), b = (int)(br % nbr);
     const int x0 = (b % nbx) * BX, y0 = ((b / nbx) % nby) * BY, z0 = (b / (nbx * nby)) * BZ;
-    __syncthreads();
-    for (int t = threadIdx.x; t < 256 * ng; t += 256) {
-      const int c8 = t % ng, v = t / ng;
-      const int x = x0 + (v & 15), y = y0 + ((v >> 4) & 3), z = z0 + (v >> 6);
-      uint4 val = make_uint4(0u, 0u, 0u, 0u);
-      if (x < a.W && y < a.H && z < a.D)
-        val = *(const uint4*)(a.g + ((((int64_t)n * a.D + z) * a.H + y) * a.W + x) * a.coutp + 8 * c8);
-      const uint32_t w4[4] = {val.x, val.y, val.z, val.w};
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        gT[8 * c8 + 2 * j][v] = (uint16_t)(w4[j] & 0xffffu);
-        gT[8 * c8 + 2 * j + 1][v] = (uint16_t)(w4[j] >> 16);
-      }
+    for (int i = 0; i < NG; i++) {
+      const int t = threadIdx.x + 256 * i, c8 = t % NG, v = t / NG;
+      const int x = x0 + (v & 15), y = y0 + ((v >> 4) & 3), z = z0 + (v >> 6);
+      gr[i] = make_uint4(0u, 0u, 0u, 0u);
+      if (c8 < ng && x < a.W && y < a.H && z < a.D)
+        gr[i] = *(const uint4*)(a.g + ((((int64_t)n * a.D + z) * a.H + y) * a.W + x) * a.coutp + 8 * c8);
     }
-    for (int t = threadIdx.x; t < (MT * 16 - a.coutp) * 256; t += 256)
-      gT[a.coutp + (t >> 8)][t & 255] = 0;
-    for (int t = threadIdx.x; t < HVOX * 2; t += 256) {
-      const int c8 = t & 1, v = t >> 1;
+#pragma unroll
+    for (int i = 0; i < NX; i++) {
+      const int t = threadIdx.x + 256 * i, c8 = t & 1, v = t >> 1;
       const int hx = v % HXs, hy = (v / HXs) % HYs, hz = v / (HXs * HYs);
       const int c = cig * 16 + 8 * c8;
-      uint4 val = make_uint4(0u, 0u, 0u, 0u);
-      if (c < a.cinp) val = load8(a.x, n, a.D, a.H, a.W, z0 + hz - 1, y0 + hy - 1, x0 + hx - 1, c);
-      const uint32_t w4[4] = {val.x, val.y, val.z, val.w};
-#pragma unroll
-      for (int dx = 0; dx < 3; dx++) {
-        const int xs = hx - dx;
-        if (xs < 0 || xs >= BX) continue;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          xT[dx][8 * c8 + 2 * j][hz][hy][xs] = (uint16_t)(w4[j] & 0xffffu);
-          xT[dx][8 * c8 + 2 * j + 1][hz][hy][xs] = (uint16_t)(w4[j] >> 16);
-        }
-      }
+      xr[i] = make_uint4(0u, 0u, 0u, 0u);
+      if (v < HVOX && c < a.cinp)
+        xr[i] = load8<POOLED>(a.x, n, a.D, a.H, a.W, z0 + hz - 1, y0 + hy - 1, x0 + hx - 1, c);
     }
+  };
+  const int sub = (row >> 2), ch = 4 * (row & 3); // voxel and channels this lane addresses
+  const bf16x8 ones = __builtin_bit_cast(bf16x8, make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u));
+  int64_t br = blockIdx.x;
+  if (br < total) load(br);
+  for (; br < total; br += gridDim.x) {
     __syncthreads();
-    if (cig == 0 && threadIdx.x < a.coutp)
-      for (int v = 0; v < 256; v++) bsum += bf2f(gT[threadIdx.x][v]);
+#pragma unroll
+    for (int i = 0; i < NG; i++) ((uint4*)gl)[threadIdx.x + 256 * i] = gr[i];
+#pragma unroll
+    for (int i = 0; i < NX; i++)
+      if (threadIdx.x + 256 * i < HVOX * 2) ((uint4*)xl)[threadIdx.x + 256 * i] = xr[i];
+    __syncthreads();
+    if (br + gridDim.x < total) load(br + gridDim.x);
 #pragma unroll
     for (int kb = 0; kb < 8; kb++) {
       // voxels 32 kb + 8 grp + j: row r = 2 kb + grp/2 (y = r % 4, z = r / 4), x = 8 (grp % 2) + j
@@ -308,18 +371,22 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradArgs a)
       const int y = r & 3, z = r >> 2;
       bf16x8 av[MT];
 #pragma unroll
-      for (int m = 0; m < MT; m++)
-        av[m] = *(const bf16x8*)&gT[m * 16 + row][32 * kb + 8 * grp];
+      for (int m = 0; m < MT; m++) {
+        const uint16_t* g0 = gl + (32 * kb + 8 * grp + sub) * GS + m * 16 + ch;
+        av[m] = join(read_tr(g0), read_tr(g0 + 4 * GS));
+      }
 #pragma unroll
       for (int j = 0; j < 7; j++) {
         const int tap = wave + 4 * j;
+        const int dz = tap / 9, dy = (tap / 3) % 3, dx = tap % 3;
+        bf16x8 bv = ones;
         if (tap < 27) {
-          const int dz = tap / 9, dy = (tap / 3) % 3, dx = tap % 3;
-          const bf16x8 bv = *(const bf16x8*)&xT[dx][row][z + dz][y + dy][xo];
-#pragma unroll
-          for (int m = 0; m < MT; m++)
-            acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], bv, acc[m][j], 0, 0, 0);
+          const uint16_t* x0 = xl + (((z + dz) * HYs + y + dy) * HXs + xo + dx + sub) * 16 + ch;
+          bv = join(read_tr(x0), read_tr(x0 + 4 * 16));
         }
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+          acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], bv, acc[m][j], 0, 0, 0);
       }
     }
   }
@@ -329,36 +396,50 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradArgs a)
 #pragma unroll
     for (int j = 0; j < 7; j++) {
       const int tap = wave + 4 * j;
-      if (tap < 27)
 #pragma unroll
-        for (int i = 0; i < 4; i++) P[((m * 16 + 4 * grp + i) * 27 + tap) * 16 + row] = acc[m][j][i];
+      for (int i = 0; i < 4; i++) {
+        if (tap < 27) P[((m * 16 + 4 * grp + i) * 27 + tap) * 16 + row] = acc[m][j][i];
+        else if (cig == 0 && row == 0)
+          a.partb[(int64_t)blockIdx.x * MT * 16 + m * 16 + 4 * grp + i] = acc[m][j][i];
+      }
     }
-  if (cig == 0 && threadIdx.x < MT * 16) a.partb[(int64_t)blockIdx.x * MT * 16 + threadIdx.x] = bsum;
 }
 
-// fixed-order sum of the partials into the FP32 gradient [co][ci][27], [co]
-__global__ void k_wgrad_reduce(const float* __restrict__ part, const float* __restrict__ partb,
-                               int nb, int ncig, int mt16, int co_n, int c0, int c0p, int c1,
-                               float* __restrict__ gw, float* __restrict__ gb)
+// Fixed-order sum of the partials into the FP32 gradient [co][ci][27], [co]:
+// kRedSlices threads of a block share the nb partials of an entry.  One thread
+// per entry left a small convolution's 14 MB to a few dozen waves, each adding
+// 512 partials one after the other: 119 us, now 6.
+constexpr int kRedSlices = 16;
+
+__global__ __launch_bounds__(64 * kRedSlices) void k_wgrad_reduce(
+    const float* __restrict__ part, const float* __restrict__ partb, int nb, int ncig, int mt16,
+    int co_n, int c0, int c0p, int c1, float* __restrict__ gw, float* __restrict__ gb)
 {
-  const int ci_n = c0 + c1;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t nw = (int64_t)co_n * ci_n * 27;
-  if (i < nw) {
-    const int tap = (int)(i % 27);
-    const int ci = (int)((i / 27) % ci_n), co = (int)(i / (27 * (int64_t)ci_n));
-    const int pci = ci < c0 ? ci : c0p + (ci - c0);
-    const int cg = pci >> 4, cl = pci & 15;
-    float s = 0.f;
-    for (int b = 0; b < nb; b++)
-      s += part[(((int64_t)b * ncig + cg) * mt16 + co) * 27 * 16 + tap * 16 + cl];
-    gw[i] = s;
-  } else if (i < nw + co_n) {
-    const int co = (int)(i - nw);
-    float s = 0.f;
-    for (int b = 0; b < nb; b++) s += partb[(int64_t)b * mt16 + co];
-    gb[co] = s;
+  __shared__ float sh[kRedSlices][64];
+  const int t = threadIdx.x & 63, slice = threadIdx.x >> 6;
+  const int percg = co_n * 27 * 16; // entries [co][tap][16] of a channel group
+  const int64_t e = (int64_t)blockIdx.x * 64 + t, nw = (int64_t)ncig * percg;
+  const bool bias = e >= nw;
+  const int cg = (int)(e / percg), in = (int)(e % percg);
+  const float* src = bias ? partb + (e - nw) : part + (int64_t)cg * mt16 * 432 + in;
+  const int64_t ld = bias ? mt16 : (int64_t)ncig * mt16 * 432;
+  float s = 0.f;
+  if (e < nw + co_n) {
+#pragma unroll 8
+    for (int b = slice; b < nb; b += kRedSlices) s += src[b * ld];
   }
+  sh[slice][t] = s;
+  __syncthreads();
+  if (slice || e >= nw + co_n) return;
+  for (int k = 1; k < kRedSlices; k++) s += sh[k][t];
+  if (bias) {
+    gb[e - nw] = s;
+    return;
+  }
+  const int cl = in & 15, tap = (in >> 4) % 27, co = in / 432, pci = cg * 16 + cl;
+  if (pci >= c0 && pci < c0p) return; // padding of the first input
+  const int ci = pci < c0 ? pci : c0 + (pci - c0p);
+  if (ci < c0 + c1) gw[((int64_t)co * (c0 + c1) + ci) * 27 + tap] = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -566,10 +647,13 @@ template <int NT>
 static void launch_conv(const ConvArgs& a, int N, hipStream_t s, int ztiles = 1)
 {
   const int cin_p = a.x.c0p + a.x.c1p;
-  const size_t halo = sizeof(uint4) * HVOX * ((cin_p < CCMAX ? cin_p : CCMAX) / 8);
+  const size_t halo = sizeof(uint4) * HVOX * ((cin_p < CCMAX ? cin_p : CCMAX) / 8) +
+                      sizeof(int) * kWhere;
   const size_t stage = a.out ? sizeof(uint16_t) * BX * BY * BZ * NT * 16 : 0;
-  k_conv<NT><<<dim3(conv_bricks(a.D, a.H, a.W), N, ztiles), 256, halo > stage ? halo : stage, s>>>(
-      a);
+  const dim3 grid(conv_bricks(a.D, a.H, a.W), N, ztiles);
+  const size_t lds = halo > stage ? halo : stage;
+  if (a.x.mode0 == 2) k_conv<NT, true><<<grid, 256, lds, s>>>(a);
+  else k_conv<NT, false><<<grid, 256, lds, s>>>(a);
 }
 
 // nt output tiles of 16 channels: one block runs all of them over its brick,
@@ -815,15 +899,18 @@ void UNet::conv_wgrad(const Conv& cv, const ConvIn& in, const uint16_t* g, int N
   a.part = wpart;
   a.partb = wpart + (int64_t)nb * ncig * mt * 16 * 27 * 16;
   const dim3 grid(nb, ncig);
+  auto run = [&](auto kernel) { kernel<<<grid, 256, 0, stream>>>(a); };
+  const bool pooled = in.mode0 == 2;
   switch (mt) {
-  case 1: k_wgrad<1><<<grid, 256, 0, stream>>>(a); break;
-  case 2: k_wgrad<2><<<grid, 256, 0, stream>>>(a); break;
-  case 3: k_wgrad<3><<<grid, 256, 0, stream>>>(a); break;
-  default: k_wgrad<4><<<grid, 256, 0, stream>>>(a); break;
+  case 1: pooled ? run(k_wgrad<1, true>) : run(k_wgrad<1, false>); break;
+  case 2: pooled ? run(k_wgrad<2, true>) : run(k_wgrad<2, false>); break;
+  case 3: pooled ? run(k_wgrad<3, true>) : run(k_wgrad<3, false>); break;
+  default: pooled ? run(k_wgrad<4, true>) : run(k_wgrad<4, false>); break;
   }
-  const int64_t nw = (int64_t)cv.co * cv.ci() * 27 + cv.co;
-  k_wgrad_reduce<<<grid1(nw), 256, 0, stream>>>(a.part, a.partb, nb, ncig, mt * 16, cv.co, cv.c0,
-                                                cv.c0p, cv.c1, grads + cv.w, grads + cv.b);
+  const unsigned nred = (unsigned)((ncig * cv.co * 432 + cv.co + 63) / 64);
+  k_wgrad_reduce<<<nred, 64 * kRedSlices, 0, stream>>>(a.part, a.partb, nb, ncig, mt * 16, cv.co,
+                                                       cv.c0, cv.c0p, cv.c1, grads + cv.w,
+                                                       grads + cv.b);
 }
 
 static ConvIn cin_of(const uint16_t* p, int c, int mode = 0, const uint16_t* p1 = nullptr, int c1 = 0)
