@@ -33,6 +33,7 @@ void launch_spmv16(Context& c, const __half* val, float scale, const float* p, f
                    bool skip_done, hipStream_t st);
 void launch_spmv16_node3(Context& c, const uint2* val, float scale, const float* p, float* q,
                          bool skip_done, hipStream_t st);
+int64_t demote16_words(const Context& c);
 int demote16_node3(Context& c, double inv_scale, uint2* out);
 
 Multigrid::~Multigrid()
@@ -1031,8 +1032,8 @@ int mg_setup(Context& c, int degree)
   IFEM_HIP(hipMemcpyAsync(m.h_lzh, m.lzh, sizeof(double), hipMemcpyDeviceToHost, c.stream));
   IFEM_HIP(hipStreamSynchronize(c.stream));
   m.kscale = m.h_lzh[0] > 0.0 ? m.h_lzh[0] : 1.0;
-  if (c.d_bcol) { // node blocks: one 8-byte load per row and neighbour in the smoother
-    if (!m.val16n) IFEM_HIP(hipMalloc(&m.val16n, sizeof(uint2) * (c.nnz > 0 ? c.nnz / 3 : 1)));
+  if (c.d_bcol) { // packs of four neighbours per row: whole words for the smoother
+    if (!m.val16n) IFEM_HIP(hipMalloc(&m.val16n, sizeof(uint2) * demote16_words(c)));
     const int rc = demote16_node3(c, 1.0 / m.kscale, m.val16n);
     if (rc) return rc;
   } else {

@@ -161,8 +161,9 @@ static int build(hipStream_t s, int n, const ShapeRows& R, int64_t entries, RowS
   IFEM_HIP(hipMemcpyAsync(&total, incl + n - 1, sizeof(int64_t), hipMemcpyDeviceToHost, s));
   IFEM_HIP(hipStreamSynchronize(s));
   if (total > entries / 8 || total > INT32_MAX) return IFEM_GPU_OK; // mostly distinct
+  // three more: the FP16 product reads the list in fours
   if (!alloc((void**)&out.start, sizeof(int32_t) * (size_t)n) ||
-      !alloc((void**)&out.table, sizeof(int32_t) * (size_t)(total > 0 ? total : 1))) {
+      !alloc((void**)&out.table, sizeof(int32_t) * (size_t)(total + 3))) {
     out.release();
     return IFEM_GPU_OK;
   }

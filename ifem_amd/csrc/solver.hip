@@ -126,12 +126,16 @@ __global__ __launch_bounds__(kThreads) void k_spmv_node3(
   if (threadIdx.x == 0) part_pq[blockIdx.x] = bs;
 }
 
-// FP16 values of a 3-component node-uniform system in node blocks: for node
-// nd and its k-th neighbour node (k < cnt, the order of bcol), 12 halfs at
-// ((rowptr[3nd]/9) + k) * 12: [row r of the node][column component j,
-// padded with a zero to 4], so that each row's three values of a neighbour
-// are one 8-byte load (instead of three 2-byte loads).  Built from the FP64
-// CSR values times inv_scale, one wave per node.
+// FP16 values of a 3-component node-uniform system: each node's three rows one
+// after the other, a row padded with zeros to whole packs of four neighbour
+// nodes (12 halfs, three 8-byte words).  Node nd starts at pack
+// pack16(r0 / 9, nd): at most 3 blocks of padding per node.
+__host__ __device__ inline int64_t pack16(int64_t blocks, int64_t nd)
+{
+  return (blocks + 3 * nd + 3) / 4;
+}
+
+// Built from the FP64 CSR values times inv_scale, one wave per node.
 __global__ void k_demote16_node3(int nnode, const int64_t* __restrict__ rowptr,
                                  const double* __restrict__ a, uint2* __restrict__ b,
                                  double inv_scale)
@@ -141,17 +145,16 @@ __global__ void k_demote16_node3(int nnode, const int64_t* __restrict__ rowptr,
   for (int nd = (int)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6); nd < nnode;
        nd += nw) {
     const int64_t r0 = rowptr[3 * nd];
-    const int cnt = (int)((rowptr[3 * nd + 1] - r0) / 3);
-    const int64_t nb = r0 / 9;
-    for (int k = lane; k < cnt; k += 64) {
+    const int len = (int)(rowptr[3 * nd + 1] - r0), words = 3 * ((len / 3 + 3) / 4);
+    uint2* dst = b + 9 * pack16(r0 / 9, nd);
+    for (int i = lane; i < 3 * words; i += 64) {
+      const int r = i / words, m = 4 * (i - r * words);
+      const double* src = a + r0 + (int64_t)r * len;
+      uint32_t h[4];
 #pragma unroll
-      for (int r = 0; r < 3; r++) {
-        const double* src = a + r0 + (int64_t)r * 3 * cnt + 3 * k;
-        const uint32_t h0 = __half_as_ushort(__float2half((float)(src[0] * inv_scale)));
-        const uint32_t h1 = __half_as_ushort(__float2half((float)(src[1] * inv_scale)));
-        const uint32_t h2 = __half_as_ushort(__float2half((float)(src[2] * inv_scale)));
-        b[(nb + k) * 3 + r] = make_uint2(h0 | (h1 << 16), h2);
-      }
+      for (int j = 0; j < 4; j++)
+        h[j] = m + j < len ? __half_as_ushort(__float2half((float)(src[m + j] * inv_scale))) : 0;
+      dst[i] = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
     }
   }
 }
@@ -159,47 +162,76 @@ __global__ void k_demote16_node3(int nnode, const int64_t* __restrict__ rowptr,
 __device__ inline float lo_half(uint32_t w) { return __half2float(__ushort_as_half((unsigned short)(w & 0xffffu))); }
 __device__ inline float hi_half(uint32_t w) { return __half2float(__ushort_as_half((unsigned short)(w >> 16))); }
 
-// q = scale * (K16 p) with the node-block FP16 values (k_demote16_node3), FP32
-// sums: the fine-level smoother's SpMV.  Same wave-per-node and XCD mapping
-// as k_spmv_node3.
+// q = scale * (K16 p) with the packed FP16 values (k_demote16_node3), FP32
+// sums: the fine-level smoother's SpMV.  Same XCD mapping as k_spmv_node3, 16
+// lanes per node, two packs of four neighbours per lane at a time.  Bound by
+// the reading of the values: elasticity 64^3 p = 2 (617 MB) 143 us, 4.3 TB/s.
+// With each row's three values of a neighbour padded to 8 bytes, one wave per
+// node: 804 MB and, with row shapes, 180 us.  8 lanes or one pack at a time:
+// 146 to 150 us.
 template <bool SKIP, bool SHAPED>
 __global__ __launch_bounds__(kThreads) void k_spmv_node3_h(
     int nnode, const int64_t* __restrict__ rowptr, const int32_t* __restrict__ start,
-    const int32_t* __restrict__ bcol, const uint2* __restrict__ val, const float* __restrict__ p,
+    const int32_t* __restrict__ cols, const uint2* __restrict__ val, const float* __restrict__ p,
     float* __restrict__ q, const double* __restrict__ scal, float scale)
 {
   if (SKIP && scal[S_DONE] != 0.0) return;
-  constexpr int WPB = kThreads / 64;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  constexpr int L = 16, U = 2, GPB = kThreads / L;
+  const int g = threadIdx.x / L, lane = threadIdx.x % L;
   const int nxcd = 8;
   const int xcd = blockIdx.x % nxcd, bl = blockIdx.x / nxcd, nbl = gridDim.x / nxcd;
   const int lo = (int)((int64_t)nnode * xcd / nxcd), hi = (int)((int64_t)nnode * (xcd + 1) / nxcd);
-  for (int nd = lo + bl * WPB + wave; nd < hi; nd += nbl * WPB) {
+  for (int nd = lo + bl * GPB + g; nd < hi; nd += nbl * GPB) {
     const int64_t r0 = rowptr[3 * nd];
-    const int cnt = (int)((rowptr[3 * nd + 1] - r0) / 3);
-    const int64_t nb = r0 / 9;
-    const int32_t* __restrict__ bc = SHAPED ? bcol + start[nd] : bcol + nb;
+    const int cnt = (int)((rowptr[3 * nd + 1] - r0) / 3), np = (cnt + 3) / 4;
+    const int32_t* __restrict__ ci = SHAPED ? cols + start[nd] : cols + r0 / 9;
     const float* __restrict__ pb = SHAPED ? p + 3 * (int64_t)nd : p;
-    const uint2* vb = val + nb * 3;
-    float s0 = 0.f, s1 = 0.f, s2 = 0.f;
-    for (int k = lane; k < cnt; k += 64) {
-      const int64_t c = 3 * (int64_t)bc[k];
-      const float x0 = pb[c], x1 = pb[c + 1], x2 = pb[c + 2];
-      const uint2 w0 = vb[3 * k], w1 = vb[3 * k + 1], w2 = vb[3 * k + 2];
-      s0 += lo_half(w0.x) * x0 + hi_half(w0.x) * x1 + lo_half(w0.y) * x2;
-      s1 += lo_half(w1.x) * x0 + hi_half(w1.x) * x1 + lo_half(w1.y) * x2;
-      s2 += lo_half(w2.x) * x0 + hi_half(w2.x) * x1 + lo_half(w2.y) * x2;
+    const uint2* __restrict__ v = val + 9 * pack16(r0 / 9, nd);
+    const int own = SHAPED ? 0 : nd; // column of the padding
+    float s[3] = {0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < np; k0 += L * U) {
+      Pack<uint2, 3> a[U][3];
+      Pack<int, 4> c[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int k = k0 + u * L + lane, m = k < np ? k : np - 1;
+        // lists are allocated with room for a whole pack behind the last entry
+        __builtin_memcpy(&c[u], ci + 4 * m, sizeof(c[u]));
+#pragma unroll
+        for (int r = 0; r < 3; r++) a[u][r] = *(const Pack<uint2, 3>*)(v + 3 * (r * np + m));
+#pragma unroll
+        for (int j = 0; j < 4; j++) c[u].v[j] = 4 * m + j < cnt ? c[u].v[j] : own;
+      }
+      Pack<float, 3> x[U][4];
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          __builtin_memcpy(&x[u][j], pb + 3 * (int64_t)c[u].v[j], sizeof(x[u][j]));
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const bool in = k0 + u * L + lane < np;
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+          float t = s[r];
+#pragma unroll
+          for (int w = 0; w < 3; w++) {
+            const uint2 h = a[u][r].v[w];
+            t += lo_half(h.x) * x[u][(4 * w) / 3].v[(4 * w) % 3];
+            t += hi_half(h.x) * x[u][(4 * w + 1) / 3].v[(4 * w + 1) % 3];
+            t += lo_half(h.y) * x[u][(4 * w + 2) / 3].v[(4 * w + 2) % 3];
+            t += hi_half(h.y) * x[u][(4 * w + 3) / 3].v[(4 * w + 3) % 3];
+          }
+          s[r] = in ? t : s[r];
+        }
+      }
     }
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-      s0 += __shfl_xor(s0, off, 64);
-      s1 += __shfl_xor(s1, off, 64);
-      s2 += __shfl_xor(s2, off, 64);
-    }
+    for (int r = 0; r < 3; r++) s[r] = group_sum<L>(s[r]);
     if (lane == 0) {
-      q[3 * nd] = s0 * scale;
-      q[3 * nd + 1] = s1 * scale;
-      q[3 * nd + 2] = s2 * scale;
+      q[3 * nd] = s[0] * scale;
+      q[3 * nd + 1] = s[1] * scale;
+      q[3 * nd + 2] = s[2] * scale;
     }
   }
 }
@@ -435,7 +467,10 @@ void launch_spmv16(Context& c, const __half* val, float scale, const float* p, f
   else launch_spmv<float, float, false, false, __half>(c, val, p, q, scale, st);
 }
 
-// The node-block FP16 copy of K / scale (3-component node-uniform systems).
+// The packed FP16 copy of K / scale (3-component node-uniform systems): its
+// size in 8-byte words, and its values.
+int64_t demote16_words(const Context& c) { return 9 * (pack16(c.nnz / 9, c.neq / 3) + 1); }
+
 int demote16_node3(Context& c, double inv_scale, uint2* out)
 {
   k_demote16_node3<<<4096, 256, 0, c.stream>>>(c.neq / 3, c.d_rowptr, c.d_val, out, inv_scale);
@@ -443,13 +478,16 @@ int demote16_node3(Context& c, double inv_scale, uint2* out)
   return IFEM_GPU_OK;
 }
 
+// Three blocks per CU (143 us; two 158, four 149, eight 155 for 64^3 p = 2).
+constexpr int kHalfGrid = 768;
+
 void launch_spmv16_node3(Context& c, const uint2* val, float scale, const float* p, float* q,
                          bool skip_done, hipStream_t st)
 {
   if (!st) st = c.stream;
   const RowShapes& sh = c.shapes;
   auto run = [&](auto kernel, const int32_t* start, const int32_t* cols) {
-    kernel<<<kGrid, kThreads, 0, st>>>(c.neq / 3, c.d_rowptr, start, cols, val, p, q, c.w.scal, scale);
+    kernel<<<kHalfGrid, kThreads, 0, st>>>(c.neq / 3, c.d_rowptr, start, cols, val, p, q, c.w.scal, scale);
   };
   if (sh.start)
     skip_done ? run(k_spmv_node3_h<true, true>, sh.start, sh.table)
@@ -510,7 +548,7 @@ int solver_setup(Context& c)
     else uniform = c.h_eq[3 * nd + 1] < 0 && c.h_eq[3 * nd + 2] < 0;
   }
   if (uniform) {
-    IFEM_HIP(hipMalloc(&c.d_bcol, sizeof(int32_t) * (c.nnz / 9 + 1)));
+    IFEM_HIP(hipMalloc(&c.d_bcol, sizeof(int32_t) * (c.nnz / 9 + 4)));
     k_build_bcol<<<c.neq / 3, 128, 0, c.stream>>>(c.neq / 3, c.d_rowptr, c.d_colind, c.d_bcol);
     IFEM_HIP(hipGetLastError());
   }
