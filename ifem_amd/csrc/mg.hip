@@ -428,46 +428,60 @@ struct DirDev {
 
 // bc = P^T (rf - qf) on the coarse grid (masked by the coarse free flags);
 // fmap: fine DOF -> vector index (-1 eliminated), nullptr for identity.
-// One thread per coarse DOF.
+// A coarse DOF sums up to kMgKC^3 fine entries, each behind its index: bound
+// by latency.  Four threads share it, one per fine plane, and a line's entries
+// are requested together.  One thread per DOF left 7 waves per CU at 34^3
+// coarse nodes: 20.2 -> 9.9 us on average over the levels of elasticity 64^3
+// p = 2.
+constexpr int kRestSplit = 4;
+
 template <int NC>
-__global__ __launch_bounds__(256) void k_mg_restrict(const float* __restrict__ rf,
-                                                     const float* __restrict__ qf,
-                                                     const int* __restrict__ fmap, Grid3 gf,
-                                                     float* __restrict__ bc,
-                                                     const unsigned char* __restrict__ cfree,
-                                                     Grid3 gc, DirDev d0, DirDev d1, DirDev d2,
-                                                     const double* __restrict__ scal)
+__global__ __launch_bounds__(64 * kRestSplit) void k_mg_restrict(
+    const float* __restrict__ rf, const float* __restrict__ qf, const int* __restrict__ fmap,
+    Grid3 gf, float* __restrict__ bc, const unsigned char* __restrict__ cfree, Grid3 gc, DirDev d0,
+    DirDev d1, DirDev d2, const double* __restrict__ scal)
 {
   if (scal && scal[S_DONE] != 0.0) return;
+  __shared__ float sh[kRestSplit][64];
   const int64_t nnc = (int64_t)gc.n0 * gc.n1 * gc.n2;
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nnc * NC) return;
-  const int64_t node = t / NC;
-  const int c = (int)(t - node * NC);
-  if (!cfree[t]) {
-    bc[t] = 0.f;
-    return;
-  }
-  const int I0 = (int)(node % gc.n0), I1 = (int)((node / gc.n0) % gc.n1);
-  const int I2 = (int)(node / ((int64_t)gc.n0 * gc.n1));
+  const int lane = threadIdx.x & 63, sub = threadIdx.x >> 6;
+  const int64_t t = (int64_t)blockIdx.x * 64 + lane;
+  const bool on = t < nnc * NC && cfree[t < nnc * NC ? t : 0];
   float acc = 0.f;
-  const int n2c = d2.ccnt[I2], n1c = d1.ccnt[I1], n0c = d0.ccnt[I0];
-  const int l2 = d2.clo[I2], l1 = d1.clo[I1], l0 = d0.clo[I0];
-  for (int kg = 0; kg < n2c; kg++) {
-    const float w2 = (float)d2.cw[(int64_t)I2 * kMgKC + kg];
-    for (int kb = 0; kb < n1c; kb++) {
-      const float w12 = w2 * (float)d1.cw[(int64_t)I1 * kMgKC + kb];
-      const int64_t frow = (int64_t)gf.n0 * ((l1 + kb) + (int64_t)gf.n1 * (l2 + kg));
-      for (int ka = 0; ka < n0c; ka++) {
-        const float w = w12 * (float)d0.cw[(int64_t)I0 * kMgKC + ka];
-        const int64_t f = (frow + l0 + ka) * NC + c;
-        const int64_t idx = fmap ? (int64_t)fmap[f] : f;
-        if (idx < 0) continue;
-        acc += w * (qf ? rf[idx] - qf[idx] : rf[idx]);
+  if (on) {
+    const int64_t node = t / NC;
+    const int c = (int)(t - node * NC);
+    const int I0 = (int)(node % gc.n0), I1 = (int)((node / gc.n0) % gc.n1);
+    const int I2 = (int)(node / ((int64_t)gc.n0 * gc.n1));
+    const int n2c = d2.ccnt[I2], n1c = d1.ccnt[I1], n0c = d0.ccnt[I0];
+    const int l2 = d2.clo[I2], l1 = d1.clo[I1], l0 = d0.clo[I0];
+    float w0[kMgKC];
+#pragma unroll
+    for (int ka = 0; ka < kMgKC; ka++)
+      w0[ka] = ka < n0c ? (float)d0.cw[(int64_t)I0 * kMgKC + ka] : 0.f;
+    for (int kg = sub; kg < n2c; kg += kRestSplit) {
+      const float w2 = (float)d2.cw[(int64_t)I2 * kMgKC + kg];
+      for (int kb = 0; kb < n1c; kb++) {
+        const float w12 = w2 * (float)d1.cw[(int64_t)I1 * kMgKC + kb];
+        const int64_t f0 = (gf.n0 * ((l1 + kb) + (int64_t)gf.n1 * (l2 + kg)) + l0) * NC + c;
+        int64_t idx[kMgKC];
+#pragma unroll
+        for (int ka = 0; ka < kMgKC; ka++)
+          idx[ka] = ka >= n0c ? -1 : fmap ? (int64_t)fmap[f0 + ka * NC] : f0 + ka * NC;
+        float v[kMgKC];
+#pragma unroll
+        for (int ka = 0; ka < kMgKC; ka++)
+          v[ka] = idx[ka] < 0 ? 0.f : qf ? rf[idx[ka]] - qf[idx[ka]] : rf[idx[ka]];
+#pragma unroll
+        for (int ka = 0; ka < kMgKC; ka++) acc += idx[ka] < 0 ? 0.f : w12 * w0[ka] * v[ka];
       }
     }
   }
-  bc[t] = acc;
+  sh[sub][lane] = acc;
+  __syncthreads();
+  if (sub || t >= nnc * NC) return;
+  for (int k = 1; k < kRestSplit; k++) acc += sh[k][lane];
+  bc[t] = acc; // 0 where eliminated
 }
 
 // xf += P xc (fine free entries only).
@@ -1171,12 +1185,12 @@ static void vcycle(Context& c, Multigrid& m, int l, const double* scal)
   const int* fmap = nullptr;
   fmap_grid(m, c, l, fmap);
   const DirDev d0 = dirdev(C.dir[0]), d1 = dirdev(C.dir[1]), d2 = dirdev(C.dir[2]);
-  const unsigned gr = grid1((int64_t)C.nnode * m.nc);
+  const unsigned gr = (unsigned)(((int64_t)C.nnode * m.nc + 63) / 64);
   if (m.nc == 3)
-    k_mg_restrict<3><<<gr, 256, 0, c.stream>>>(L.r, L.q, fmap, grid_of(L), C.b, C.freem, grid_of(C),
+    k_mg_restrict<3><<<gr, 64 * kRestSplit, 0, c.stream>>>(L.r, L.q, fmap, grid_of(L), C.b, C.freem, grid_of(C),
                                                d0, d1, d2, scal);
   else
-    k_mg_restrict<1><<<gr, 256, 0, c.stream>>>(L.r, L.q, fmap, grid_of(L), C.b, C.freem, grid_of(C),
+    k_mg_restrict<1><<<gr, 64 * kRestSplit, 0, c.stream>>>(L.r, L.q, fmap, grid_of(L), C.b, C.freem, grid_of(C),
                                                d0, d1, d2, scal);
   vcycle(c, m, l + 1, scal);
   if (m.nc == 3)
