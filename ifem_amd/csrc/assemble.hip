@@ -335,6 +335,13 @@ __device__ inline void gp_geometry_at(ConstArgs& a, int64_t id, bool want_rhs)
     const double dV = 0.125 * (a.span1[e1] * a.span2[e2] * a.span3[e3]);
     wdet = det * (dV * a.gw[q1] * a.gw[q2] * a.gw[q3]);
   }
+  if ((VEC || a.ncomp == 3) && a.geo_pairs) {
+    double2* out = reinterpret_cast<double2*>(a.gp_geo) + e * gp3 * (GeoRec<3>::N / 2) + q;
+#pragma unroll
+    for (int k = 0; k < 4; k++) out[k * gp3] = make_double2(Ji[2 * k], Ji[2 * k + 1]);
+    out[4 * gp3] = make_double2(Ji[8], wdet);
+    return;
+  }
   if (VEC || a.ncomp == 3) {
     double* out = a.gp_geo + e * gp3 * GeoRec<3>::N + q;
 #pragma unroll
@@ -810,6 +817,12 @@ int& asm_half_slot(Context& c, int p, int ng, int nc, bool fp32)
   return c.asm_half[p][ng > p + 1 ? 1 : 0][nc == 3 ? 1 : 0][fp32 ? 1 : 0];
 }
 
+// Vector problems that the direct line kernels assemble (lines2.hip, lines3.hip).
+static bool direct_lines(int p, int ng, bool fp32)
+{
+  return p == 3 || (p == 2 && (ng == 4 || fp32));
+}
+
 // The line kernels of degree p with ng Gauss points per direction
 // (lines1.hip .. lines3.hip).
 static int launch_lines(Context& c, const AsmArgs& args, int p, int ng, bool fp32, bool has_rhs)
@@ -899,6 +912,7 @@ static int assemble_p(Context& c, const SysView& sv, const PatchRec& Pt, const i
     c.gpgeo_cap = need;
   }
   a.gp_geo = c.d_gpgeo;
+  a.geo_pairs = c.ncomp == 3 && direct_lines(P, ng, fp32);
   if (!c.d_asmargs) IFEM_HIP(hipMalloc(&c.d_asmargs, sizeof(AsmArgs)));
   IFEM_HIP(hipMemcpyAsync(c.d_asmargs, &a, sizeof(AsmArgs), hipMemcpyHostToDevice, c.stream));
   IFEM_HIP(hipEventRecord(c.ev0, c.stream));

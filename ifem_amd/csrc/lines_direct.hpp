@@ -310,11 +310,22 @@ __device__ __forceinline__ void line_impl(
         // element by k_gp_geometry: J^-1 and w*detJ (vector), or
         // M = w*detJ*kappa*J^-1 J^-T and w*detJ*f (scalar)
         const int64_t ge = (int64_t)e1 + (int64_t)a.nel1 * (e2 + (int64_t)a.nel2 * e3);
-        const double* __restrict__ rec = a.gp_geo + ge * (GP3 * GeoRec<NC>::N) + q;
         T R[GeoRec<NC>::N];
+        if constexpr (NC == 3) {
+          const double2* __restrict__ rec =
+              reinterpret_cast<const double2*>(a.gp_geo) + ge * (GP3 * (GeoRec<NC>::N / 2)) + q;
 #pragma unroll
-        for (int k = 0; k < GeoRec<NC>::N; k++)
-          R[k] = NC == 1 && k == 6 && !HAS_RHS ? T(0) : (T)rec[k * GP3];
+          for (int k = 0; k < GeoRec<NC>::N / 2; k++) {
+            const double2 v = rec[k * GP3];
+            R[2 * k] = (T)v.x;
+            R[2 * k + 1] = (T)v.y;
+          }
+        } else {
+          const double* __restrict__ rec = a.gp_geo + ge * (GP3 * GeoRec<NC>::N) + q;
+#pragma unroll
+          for (int k = 0; k < GeoRec<NC>::N; k++)
+            R[k] = k == 6 && !HAS_RHS ? T(0) : (T)rec[k * GP3];
+        }
         if (NC == 3) {
 #pragma unroll
           for (int m = 0; m < 9; m++) geo[t][m] = R[m];
