@@ -62,14 +62,14 @@ constexpr int line_row_stride(int n)
 
 template <int P, int NG, int NC>
 struct LineCfg {
+  static_assert(P <= 2, "the direction-2 factors and T2 of a unit are held in registers");
   static constexpr int P1 = P + 1, W1 = 2 * P + 1, WW = W1 * W1, WN = W1 * WW;
   static constexpr int GP3 = NG * NG * NG;
   // slots: component pairs, or lines per workgroup (as many as fill the
   // workgroup's units and column threads about equally)
   static constexpr int SL = NC == 3 ? 9
                             : P == 1 ? (NG == 2 ? 12 : 8)
-                            : P == 2 ? (NG == 3 ? 8 : 6)
-                                     : (NG == 4 ? 5 : 4);
+                                     : 8;
   static constexpr int NL = NC == 3 ? 1 : SL;     // lines per workgroup (most)
   static constexpr int NU = NG * 9 * SL;          // units
   static constexpr int NR = NG * NL;              // right-hand side units
@@ -78,17 +78,10 @@ struct LineCfg {
   static constexpr int Q2 = P1 * NG;              // points per line in direction 2
   static constexpr int NE2 = NL + P;              // elements in direction 2
   static constexpr int NQ2 = NE2 * NG;
-  static constexpr int Q3C = P < 3 ? NG : 2;      // q3 points per chunk
-  static constexpr int NCH = (NG + Q3C - 1) / Q3C; // chunks per element row e3
-  static constexpr int RS = line_row_stride(Q3C * NQ2);
+  static constexpr int RS = line_row_stride(NG * NQ2);
   static constexpr int NROW = NC == 3 ? 3 : NL;   // rows per line position
   static constexpr int NCOL = WN * NC;            // columns of a full row
-  static constexpr int GPC = NG * NG * Q3C;       // points per element and chunk
-  // exchange: T2 rows dk per pass, odd stride per unit
-  static constexpr int DKP = P < 3 ? W1 : (NC == 3 && NG == 4 ? W1 : 4);
-  static constexpr int NPASS = (W1 + DKP - 1) / DKP;
-  static constexpr int ES = DKP * W1 | 1;
-  static constexpr bool C2REG = P < 3;            // direction-2 factors in registers
+  static constexpr int ES = WW | 1;               // exchange: odd stride per unit
 };
 
 template <int P, int NG, int NC, typename T, bool RHS>
@@ -102,7 +95,6 @@ struct LineShared {
   alignas(16) T buf[line_max(2 * CHUNK, EX)];
   alignas(16) double row[C::SL * C::WN]; // complete rows, per column line and slot
   alignas(16) T c3[5][C::P1 * NG][C::P1];
-  alignas(16) T c2[C::C2REG ? 1 : C::NL * 5 * C::Q2][C::P1];
   double rrow[C::NL];
   int64_t base[C::NROW];
   int req[C::NROW], full[C::NROW];
@@ -178,35 +170,26 @@ __device__ __forceinline__ void line_group(ConstArgs& a, const int j0, const int
     const int m = g / NG, e = kc - P + m;
     sh.c3[v][g][b] = e >= 0 && e < a.nel3 ? factor(a.tabN3, a.tabD3, e, g % NG, m, b, v) : T(0);
   }
-  T c2r[C::C2REG ? C::Q2 : 1][P1];
-  if constexpr (C::C2REG) {
+  T c2r[C::Q2][P1];
 #pragma unroll
-    for (int g = 0; g < C::Q2; g++) {
-      const int m = g / NG, e = j0 + lj - P + m;
-      const bool ok = lj < nl && e >= 0 && e < a.nel2;
+  for (int g = 0; g < C::Q2; g++) {
+    const int m = g / NG, e = j0 + lj - P + m;
+    const bool ok = lj < nl && e >= 0 && e < a.nel2;
 #pragma unroll
-      for (int b = 0; b < P1; b++) c2r[g][b] = ok ? factor(a.tabN2, a.tabD2, e, g % NG, m, b, v2) : T(0);
-    }
-  } else {
-    for (int t = tid; t < NL * 5 * C::Q2 * P1; t += TH) {
-      const int b = t % P1, g = (t / P1) % C::Q2, lv = t / (P1 * C::Q2), v = lv % 5, l = lv / 5;
-      const int m = g / NG, e = j0 + l - P + m;
-      sh.c2[lv * C::Q2 + g][b] =
-          l < nl && e >= 0 && e < a.nel2 ? factor(a.tabN2, a.tabD2, e, g % NG, m, b, v) : T(0);
-    }
+    for (int b = 0; b < P1; b++) c2r[g][b] = ok ? factor(a.tabN2, a.tabD2, e, g % NG, m, b, v2) : T(0);
   }
 
   // ---- Gauss-point loader: the items (element m2, component, point) of a
-  // chunk (element row m3, part h of its q3 points); the next chunk's are
+  // chunk (element row m3); the next chunk's are
   // loaded into registers while the current one is used
   constexpr int NLC = NC == 3 ? (RHS ? 10 : 9) : NCOMP; // loaded components
-  constexpr int NIT = C::NE2 * NLC * C::GPC;
+  constexpr int NIT = C::NE2 * NLC * C::GP3;
   constexpr int NI = (NIT + TH - 1) / TH;
   int goff[NI], dst[NI];
 #pragma unroll
   for (int n = 0; n < NI; n++) {
     const int it = tid + n * TH;
-    const int g = it % C::GPC, c = (it / C::GPC) % NLC, m2 = it / (C::GPC * NLC);
+    const int g = it % C::GP3, c = (it / C::GP3) % NLC, m2 = it / (C::GP3 * NLC);
     const int e2 = j0 - P + m2;
     const int g1 = g % NG, g2 = (g / NG) % NG, g3 = g / (NG * NG);
     const bool ok = it < NIT && m2 < nl + P && e2 >= 0 && e2 < a.nel2;
@@ -215,18 +198,16 @@ __device__ __forceinline__ void line_group(ConstArgs& a, const int j0, const int
     dst[n] = it < NIT ? (cl * NG + g1) * C::RS + g3 * C::NQ2 + m2 * NG + g2 : -1;
   }
   double pv[NI], pw[NC == 3 ? NI : 1];
-  auto load_chunk = [&](int e1, int m3, int h) {
+  auto load_chunk = [&](int e1, int m3) {
     const double* __restrict__ src =
         a.gp_geo +
-        ((int64_t)e1 + (int64_t)a.nel1 * ((j0 - P) + (int64_t)a.nel2 * (kc - P + m3))) * (RN * C::GP3) +
-        h * C::GPC;
+        ((int64_t)e1 + (int64_t)a.nel1 * ((j0 - P) + (int64_t)a.nel2 * (kc - P + m3))) * (RN * C::GP3);
 #pragma unroll
     for (int n = 0; n < NI; n++) {
       const int it = tid + n * TH;
-      // the last part of an odd number of q3 points is shorter
-      const bool ok = goff[n] >= 0 && (NG % C::Q3C == 0 || h * C::Q3C + (it % C::GPC) / (NG * NG) < NG);
+      const bool ok = goff[n] >= 0;
       pv[n] = ok ? src[goff[n]] : 0.0;
-      if constexpr (NC == 3) pw[n] = ok ? src[goff[n] + (9 - (it / C::GPC) % NLC) * C::GP3] : 0.0;
+      if constexpr (NC == 3) pw[n] = ok ? src[goff[n] + (9 - (it / C::GP3) % NLC) * C::GP3] : 0.0;
     }
   };
   auto store_chunk = [&](T* __restrict__ cb) {
@@ -234,7 +215,7 @@ __device__ __forceinline__ void line_group(ConstArgs& a, const int j0, const int
     for (int n = 0; n < NI; n++) {
       if (NIT % TH != 0 && dst[n] < 0) continue;
       if constexpr (NC == 3) {
-        const bool wc = RHS && ((tid + n * TH) / C::GPC) % NLC == 9;
+        const bool wc = RHS && ((tid + n * TH) / C::GP3) % NLC == 9;
         cb[dst[n]] = wc ? (T)pw[n] : (T)pw[n] * (T)pv[n];
         cb[dst[n] + (wc ? NG * C::RS : 9 * NG * C::RS)] = wc ? T(1) : (T)pv[n];
       } else {
@@ -245,62 +226,28 @@ __device__ __forceinline__ void line_group(ConstArgs& a, const int j0, const int
 
   // ---- unit sums of one chunk
   T t2[W1][W1];
-  auto units = [&](const T* __restrict__ cb, auto m3c, auto hc) {
-    constexpr int m3 = decltype(m3c)::value, h = decltype(hc)::value;
-    constexpr int NQ = NG - h * C::Q3C < C::Q3C ? NG - h * C::Q3C : C::Q3C;
+  auto units = [&](const T* __restrict__ cb, auto m3c) {
+    constexpr int m3 = decltype(m3c)::value;
     const T* __restrict__ A = cb + oA;
     const T* __restrict__ B = cb + oB;
-    if constexpr (C::C2REG) {
 #pragma unroll
-      for (int q3 = 0; q3 < NQ; q3++) {
-        T t1[W1];
+    for (int q3 = 0; q3 < NG; q3++) {
+      T t1[W1];
 #pragma unroll
-        for (int d = 0; d < W1; d++) t1[d] = T(0);
+      for (int d = 0; d < W1; d++) t1[d] = T(0);
 #pragma unroll
-        for (int g = 0; g < C::Q2; g++) {
-          T v = A[q3 * C::NQ2 + g];
-          if (NC == 3) v *= B[q3 * C::NQ2 + g];
+      for (int g = 0; g < C::Q2; g++) {
+        T v = A[q3 * C::NQ2 + g];
+        if (NC == 3) v *= B[q3 * C::NQ2 + g];
 #pragma unroll
-          for (int b = 0; b < P1; b++) t1[g / NG + b] += v * c2r[g][b];
-        }
-#pragma unroll
-        for (int b = 0; b < P1; b++) {
-          const T f = sh.c3[v3][m3 * NG + h * C::Q3C + q3][b];
-#pragma unroll
-          for (int d = 0; d < W1; d++) t2[m3 + b][d] += f * t1[d];
-        }
-      }
-    } else {
-      T t1[NQ][W1];
-#pragma unroll
-      for (int q3 = 0; q3 < NQ; q3++)
-#pragma unroll
-        for (int d = 0; d < W1; d++) t1[q3][d] = T(0);
-      const T(*__restrict__ F)[P1] = &sh.c2[(lj * 5 + v2) * C::Q2];
-#pragma unroll
-      for (int m2 = 0; m2 < P1; m2++) {
-#pragma unroll
-        for (int q2 = 0; q2 < NG; q2++) {
-          T f[P1];
-#pragma unroll
-          for (int b = 0; b < P1; b++) f[b] = F[m2 * NG + q2][b];
-#pragma unroll
-          for (int q3 = 0; q3 < NQ; q3++) {
-            T v = A[q3 * C::NQ2 + m2 * NG + q2];
-            if (NC == 3) v *= B[q3 * C::NQ2 + m2 * NG + q2];
-#pragma unroll
-            for (int b = 0; b < P1; b++) t1[q3][m2 + b] += v * f[b];
-          }
-        }
+        for (int b = 0; b < P1; b++) t1[g / NG + b] += v * c2r[g][b];
       }
 #pragma unroll
-      for (int q3 = 0; q3 < NQ; q3++)
+      for (int b = 0; b < P1; b++) {
+        const T f = sh.c3[v3][m3 * NG + q3][b];
 #pragma unroll
-        for (int b = 0; b < P1; b++) {
-          const T f = sh.c3[v3][m3 * NG + h * C::Q3C + q3][b];
-#pragma unroll
-          for (int d = 0; d < W1; d++) t2[m3 + b][d] += f * t1[q3][d];
-        }
+        for (int d = 0; d < W1; d++) t2[m3 + b][d] += f * t1[d];
+      }
     }
   };
 
@@ -317,12 +264,11 @@ __device__ __forceinline__ void line_group(ConstArgs& a, const int j0, const int
     for (int d = 0; d < W1; d++) sw[r][d] = 0.0;
     rw[r] = 0.0;
   }
-  auto columns = [&](int e1, int d0) {
+  auto columns = [&](int e1) {
     ConstTable tn = (ConstTable)a.tabN1 + (int64_t)e1 * NG * P1;
     ConstTable td = (ConstTable)a.tabD1 + (int64_t)e1 * NG * P1;
-    const int dk = cd / W1;
-    if (tid < C::NCT && (C::NPASS == 1 || (dk >= d0 && dk < d0 + C::DKP))) {
-      const T* __restrict__ E = sh.buf + cs * C::ES + cd - d0 * W1;
+    if (tid < C::NCT) {
+      const T* __restrict__ E = sh.buf + cs * C::ES + cd;
 #pragma unroll
       for (int q = 0; q < NG; q++) {
         const T* __restrict__ Eq = E + q * 9 * SL * C::ES;
@@ -345,8 +291,8 @@ __device__ __forceinline__ void line_group(ConstArgs& a, const int j0, const int
         }
       }
     }
-    if (RHS && tid < NL && P >= d0 && P < d0 + C::DKP) {
-      const T* __restrict__ E = sh.buf + (C::NU + tid) * C::ES + (P - d0) * W1 + P;
+    if (RHS && tid < NL) {
+      const T* __restrict__ E = sh.buf + (C::NU + tid) * C::ES + P * W1 + P;
 #pragma unroll
       for (int q = 0; q < NG; q++) {
         const double m = E[q * NL * C::ES];
@@ -482,7 +428,7 @@ __device__ __forceinline__ void line_group(ConstArgs& a, const int j0, const int
   const int eb = i1 < a.nel1 ? i1 : a.nel1;          // past their last layer
   int rq = rthread ? a.eq[rdof0 + (int64_t)ea * NC] : -1, rqn = -1;
   int buf = 0;
-  load_chunk(ea, mlo, 0);
+  load_chunk(ea, mlo);
   store_chunk(sh.buf);
 #pragma unroll 1
   for (int i = ea; i < i1; i++) {
@@ -503,43 +449,30 @@ __device__ __forceinline__ void line_group(ConstArgs& a, const int j0, const int
       // the current chunk is in buffer buf; the next chunk of the layer goes
       // to the other one, the next layer's first chunk stays in registers
       // until the exchange over the buffers is over
-      auto part = [&](auto m3c, auto hc) {
-        constexpr int m3 = decltype(m3c)::value, h = decltype(hc)::value;
-        line_barrier();
-        const bool more = h + 1 < C::NCH || m3 < mhi;
-        if (h + 1 < C::NCH) load_chunk(i, m3, h + 1);
-        else if (m3 < mhi) load_chunk(i, m3 + 1, 0);
-        else if (i + 1 < eb) load_chunk(i + 1, mlo, 0);
-        units(sh.buf + buf * S::CHUNK, m3c, hc);
-        buf ^= 1;
-        if (more) store_chunk(sh.buf + buf * S::CHUNK);
-      };
       auto row3 = [&](auto m3c) {
         constexpr int m3 = decltype(m3c)::value;
         if (m3 < mlo || m3 > mhi) return;
-        part(m3c, std::integral_constant<int, 0>{});
-        if constexpr (C::NCH > 1) part(m3c, std::integral_constant<int, 1>{});
-        if constexpr (C::NCH > 2) part(m3c, std::integral_constant<int, 2>{});
+        line_barrier();
+        const bool more = m3 < mhi;
+        if (more) load_chunk(i, m3 + 1);
+        else if (i + 1 < eb) load_chunk(i + 1, mlo);
+        units(sh.buf + buf * S::CHUNK, m3c);
+        buf ^= 1;
+        if (more) store_chunk(sh.buf + buf * S::CHUNK);
       };
       row3(std::integral_constant<int, 0>{});
       row3(std::integral_constant<int, 1>{});
       if constexpr (P >= 2) row3(std::integral_constant<int, 2>{});
-      if constexpr (P >= 3) row3(std::integral_constant<int, 3>{});
       // exchange (over the chunk buffers) and direction 1
-      auto pass = [&](auto pc) {
-        constexpr int d0 = decltype(pc)::value * C::DKP;
-        line_barrier();
-        if (unit) {
+      line_barrier();
+      if (unit) {
 #pragma unroll
-          for (int k = d0; k < W1 && k < d0 + C::DKP; k++)
+        for (int k = 0; k < W1; k++)
 #pragma unroll
-            for (int d = 0; d < W1; d++) sh.buf[tid * C::ES + (k - d0) * W1 + d] = t2[k][d];
-        }
-        line_barrier();
-        columns(i, d0);
-      };
-      pass(std::integral_constant<int, 0>{});
-      if constexpr (C::NPASS > 1) pass(std::integral_constant<int, 1>{});
+          for (int d = 0; d < W1; d++) sh.buf[tid * C::ES + k * W1 + d] = t2[k][d];
+      }
+      line_barrier();
+      columns(i);
     }
     const bool out = i >= i0;
     if (out) {
