@@ -37,6 +37,7 @@
 // results are bitwise reproducible.
 #pragma once
 
+#include <cstdint>
 #include <type_traits>
 
 #include "asmargs.hpp"
@@ -82,6 +83,15 @@ struct LineCfg {
   static constexpr int NROW = NC == 3 ? 3 : NL;   // rows per line position
   static constexpr int NCOL = WN * NC;            // columns of a full row
   static constexpr int ES = WW | 1;               // exchange: odd stride per unit
+  // offsets of a group's records in 64 bits (WIDE): where NE2 elements of
+  // direction 2 lie 2^31 values apart.  In 32 bits elsewhere: the wider
+  // offsets cost vector problems of degree 2 with a body force their second
+  // wave per SIMD (249 -> 256 registers and more)
+  static constexpr bool wide(int nel1)
+  {
+    constexpr int64_t rec = (int64_t)GeoRec<NC>::N * GP3;
+    return ((int64_t)(NE2 - 1) * nel1 + 1) * rec > INT32_MAX;
+  }
 };
 
 template <int P, int NG, int NC, typename T, bool RHS>
@@ -125,7 +135,8 @@ __device__ __forceinline__ int window_eq(ConstArgs& a, int i, int jc, int kc, in
 }
 
 // ACCUM: the rows are shared with other patches, values are added to them.
-template <int P, int NG, int NC, typename T, bool RHS, bool ACCUM>
+// WIDE: see LineCfg::wide.
+template <int P, int NG, int NC, typename T, bool RHS, bool ACCUM, bool WIDE>
 __device__ __forceinline__ void line_group(ConstArgs& a, const int j0, const int nl, const int kc,
                                            const int i0, const int i1,
                                            LineShared<P, NG, NC, T, RHS>& sh)
@@ -185,7 +196,9 @@ __device__ __forceinline__ void line_group(ConstArgs& a, const int j0, const int
   constexpr int NLC = NC == 3 ? (RHS ? 10 : 9) : NCOMP; // loaded components
   constexpr int NIT = C::NE2 * NLC * C::GP3;
   constexpr int NI = (NIT + TH - 1) / TH;
-  int goff[NI], dst[NI];
+  using Offset = std::conditional_t<WIDE, int64_t, int>;
+  Offset goff[NI];
+  int dst[NI];
 #pragma unroll
   for (int n = 0; n < NI; n++) {
     const int it = tid + n * TH;
@@ -193,7 +206,7 @@ __device__ __forceinline__ void line_group(ConstArgs& a, const int j0, const int
     const int e2 = j0 - P + m2;
     const int g1 = g % NG, g2 = (g / NG) % NG, g3 = g / (NG * NG);
     const bool ok = it < NIT && m2 < nl + P && e2 >= 0 && e2 < a.nel2;
-    goff[n] = ok ? (m2 * a.nel1 * RN + c) * C::GP3 + g : -1;
+    goff[n] = ok ? ((Offset)m2 * a.nel1 * RN + c) * C::GP3 + g : -1;
     const int cl = NC == 3 && c == 9 ? 18 : c;
     dst[n] = it < NIT ? (cl * NG + g1) * C::RS + g3 * C::NQ2 + m2 * NG + g2 : -1;
   }
@@ -507,7 +520,7 @@ __device__ __forceinline__ void line_group(ConstArgs& a, const int j0, const int
 // Rows of one group of lines: the lines [j0, j0 + nl) at k and the segment
 // [i0, i1) of their rows, from the group's index (segment fastest, then line
 // group, then k).
-template <int P, int NG, int NC, typename T, bool RHS, bool ACCUM>
+template <int P, int NG, int NC, typename T, bool RHS, bool ACCUM, bool WIDE>
 __global__ __launch_bounds__((LineCfg<P, NG, NC>::TH), ACCUM ? 2 : 1) void k_lines(const AsmArgs* __restrict__ args,
                                                                     int ngj, int nseg, int total)
 {
@@ -521,14 +534,14 @@ __global__ __launch_bounds__((LineCfg<P, NG, NC>::TH), ACCUM ? 2 : 1) void k_lin
   const int seg = g % nseg, jg = (g / nseg) % ngj, kc = g / (nseg * ngj);
   const int j0 = (int)((int64_t)a.n2 * jg / ngj), j1 = (int)((int64_t)a.n2 * (jg + 1) / ngj);
   const int i0 = (int)((int64_t)a.n1 * seg / nseg), i1 = (int)((int64_t)a.n1 * (seg + 1) / nseg);
-  line_group<P, NG, NC, T, RHS, ACCUM>(a, j0, j1 - j0, kc, i0, i1, sh);
+  line_group<P, NG, NC, T, RHS, ACCUM, WIDE>(a, j0, j1 - j0, kc, i0, i1, sh);
 }
 
 // Batch of scalar patches: persistent workgroups take the next item of the
 // degree's list (largest first) from its queue counter.  An item's rows are
 // written by one workgroup and their sums do not depend on the split, so
 // results do not depend on which workgroup takes which item.
-template <int P, typename T, bool RHS>
+template <int P, typename T, bool RHS, bool WIDE>
 __global__ __launch_bounds__((LineCfg<P, P + 1, 1>::TH), 2) void k_lines_batch(
     const AsmArgs* __restrict__ args, const LineItem* __restrict__ items, int nitems,
     int* __restrict__ queue)
@@ -541,7 +554,7 @@ __global__ __launch_bounds__((LineCfg<P, P + 1, 1>::TH), 2) void k_lines_batch(
     const int it = __builtin_amdgcn_readfirstlane(next);
     if (it >= nitems) break;
     const LineItem w = items[it];
-    line_group<P, P + 1, 1, T, RHS, false>(const_args(args)[w.patch], w.j0, w.nl, w.k, w.i0, w.i1, sh);
+    line_group<P, P + 1, 1, T, RHS, false, WIDE>(const_args(args)[w.patch], w.j0, w.nl, w.k, w.i0, w.i1, sh);
     __syncthreads();
   }
 }

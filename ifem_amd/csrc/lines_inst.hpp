@@ -39,19 +39,26 @@ static int row_segments(int n1, int p, int64_t groups, int res, int ncu)
   return best;
 }
 
-template <int P, int NG, int NC, typename T, bool RHS, bool ACCUM>
-static int launch_lines_a(Context& c, const AsmArgs& a, int variant)
+template <int P, int NG, int NC, typename T, bool RHS, bool ACCUM, bool WIDE>
+static int launch_lines_w(Context& c, const AsmArgs& a, int variant)
 {
   using C = LineCfg<P, NG, NC>;
-  static const int res = resident_blocks(k_lines<P, NG, NC, T, RHS, ACCUM>, C::TH);
+  static const int res = resident_blocks(k_lines<P, NG, NC, T, RHS, ACCUM, WIDE>, C::TH);
   const int ngj = (a.n2 + C::NL - 1) / C::NL;
   int nseg = variant == 2 ? 1 : row_segments(a.n1, P, (int64_t)ngj * a.n3, res, 256);
   if (variant == 1) nseg = std::min(2 * nseg, a.n1);
   const int total = ngj * a.n3 * nseg;
-  k_lines<P, NG, NC, T, RHS, ACCUM><<<(total + 7) / 8 * 8, C::TH, 0, c.stream>>>(
+  k_lines<P, NG, NC, T, RHS, ACCUM, WIDE><<<(total + 7) / 8 * 8, C::TH, 0, c.stream>>>(
       static_cast<const AsmArgs*>(c.d_asmargs), ngj, nseg, total);
   IFEM_HIP(hipGetLastError());
   return IFEM_GPU_OK;
+}
+
+template <int P, int NG, int NC, typename T, bool RHS, bool ACCUM>
+static int launch_lines_a(Context& c, const AsmArgs& a, int variant)
+{
+  return LineCfg<P, NG, NC>::wide(a.nel1) ? launch_lines_w<P, NG, NC, T, RHS, ACCUM, true>(c, a, variant)
+                                          : launch_lines_w<P, NG, NC, T, RHS, ACCUM, false>(c, a, variant);
 }
 
 template <int P, int NG, int NC, typename T, bool RHS>
@@ -76,16 +83,27 @@ static int launch_lines_ng(Context& c, const AsmArgs& a, bool fp32, bool rhs, in
                       : launch_lines_nc<P, NG, 3>(c, a, fp32, rhs, variant);
 }
 
+template <int P, typename T, bool RHS, bool WIDE>
+static int launch_batch_w(Context& c, const AsmArgs* args, const LineItem* items, int n, int* queue,
+                          int ncu)
+{
+  using C = LineCfg<P, P + 1, 1>;
+  static const int res = resident_blocks(k_lines_batch<P, T, RHS, WIDE>, C::TH);
+  k_lines_batch<P, T, RHS, WIDE><<<std::max(1, std::min(n, res * ncu)), C::TH, 0, c.stream>>>(
+      args, items, n, queue);
+  IFEM_HIP(hipGetLastError());
+  return IFEM_GPU_OK;
+}
+
 template <int P, typename T, bool RHS>
 static int launch_batch_t(Context& c, const AsmArgs* args, const LineItem* items, int n, int* queue,
                           int ncu)
 {
-  using C = LineCfg<P, P + 1, 1>;
-  static const int res = resident_blocks(k_lines_batch<P, T, RHS>, C::TH);
-  k_lines_batch<P, T, RHS><<<std::max(1, std::min(n, res * ncu)), C::TH, 0, c.stream>>>(args, items, n,
-                                                                                     queue);
-  IFEM_HIP(hipGetLastError());
-  return IFEM_GPU_OK;
+  bool wide = false;
+  for (const BatchPatch& bp : c.batch->pp)
+    wide |= bp.p == P && LineCfg<P, P + 1, 1>::wide(c.patches[bp.patch].nel[0]);
+  return wide ? launch_batch_w<P, T, RHS, true>(c, args, items, n, queue, ncu)
+              : launch_batch_w<P, T, RHS, false>(c, args, items, n, queue, ncu);
 }
 
 } // namespace ifem
