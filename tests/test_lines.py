@@ -55,3 +55,27 @@ def test_lines_match_oracle(nc, p, nel, fix):
     assert np.max(np.abs(gA - A)) <= 1e-12 * np.max(np.abs(A))
     assert np.max(np.abs(gb - b)) <= 1e-12 * max(np.max(np.abs(b)), 1e-300)
     assert np.max(np.abs(A32 - A)) <= 1e-5 * np.max(np.abs(A))
+
+
+@pytest.mark.parametrize("nel", [(1, 1, 1), (5, 5, 5), (8, 3, 2), (29, 4, 3), (64, 2, 2)],
+                         ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("nc,p,ng", [(1, 1, 2), (1, 1, 3), (1, 2, 3), (3, 1, 2), (3, 1, 3), (3, 2, 3)])
+def test_row_splits_give_the_same_bits(nc, p, ng, nel):
+    """Variants 0 (the built-in rule: down to one row per segment on small
+    patches), 1 (twice as many segments) and 2 (whole lines)."""
+    pb = _problem(nc, p, nel, "none")
+    print(f"[gpu] row splits nc={nc} p={p} ng={ng} nel={nel}", flush=True)
+    out = []
+    with Session() as s:
+        s.bind(s.add_patch(pb.patch), nc, pb.meqn, pb.neq)
+        s.init_assembly()
+        for variant in (-1, 0, 1, 2):
+            for precision in (FP64, FP32):
+                if (nc, p, precision) != (3, 2, FP32):  # a kernel without row segments
+                    s.set_assembly_variant(p, ng, nc, precision, variant)
+                s.assemble(pb.integrand, (ng,) * 3, precision)
+            _, _, A, b = s.system()
+            out.append((A.copy(), b.copy(), s.values_fp32().copy()))
+    for got in out[1:]:
+        for x, y in zip(out[0], got):
+            assert np.array_equal(x, y)
