@@ -47,7 +47,7 @@ __device__ inline double bspmv_rows(int r0, int r1, const int64_t* __restrict__ 
     const int64_t b = rowptr[row];
     const int cnt = (int)(rowptr[row + 1] - b);
     const int32_t* __restrict__ ci = SHAPED ? colind + start[row] : colind + b;
-    const ACC s = group_sum<L>(row_dot<L, ACC>(l, cnt, val + b, ci, SHAPED ? p + row : p));
+    const ACC s = group_sum<L>(row_dot<L, 4, ACC>(l, cnt, val + b, ci, SHAPED ? p + row : p));
     if (l == 0) {
       q[row] = (V)s;
       if (DOT) pq += (double)((ACC)p[row] * s);

@@ -34,21 +34,21 @@
 
 namespace ifem {
 
-constexpr int kRowLanes = 8, kNodeLanes = 16; // lanes of the products per row, per node
-constexpr int kUpd = 512;                     // threads of the update kernels
+constexpr int kUpd = 512; // threads of the update kernels
 
 // ---------------------------------------------------------------------------
-// SpMV q = A p (CSR), 8 lanes per row; with DOT, per-block partial <p,q>.
+// SpMV q = A p (CSR), L lanes per row, 2 L U entries of it in a round; with
+// DOT, per-block partial <p,q>.
 // SKIP: return at once when scal[S_DONE] is set (work queued past convergence).
 // VV: type of the stored values (V, or FP16 values scaled by 1/scale).
 // SHAPED: columns from the row shapes (start per row, table `cols`).
-// Bound by the reading of the values.  8 lanes of two entries and four steps
-// ahead take a row of 125 in one round with three butterfly steps; one wave
-// per row spent its time in the six steps of its sum and waited for two loads
-// at a time.  Diffusion 48^3 p = 2 FP64 (14.5 M entries, resident in the last
-// level cache): 29.3 -> 20 us, of which the shapes' 8 B per entry instead of
-// 12 give a third.
-template <typename V, typename ACC, bool DOT, bool SKIP = DOT, typename VV = V, bool SHAPED = false>
+// Bound by the reading of the values, and on small systems by the latency of a
+// row's rounds (product_lanes has the choices).  8 lanes of four pairs take a
+// row of 125 in two rounds with three butterfly steps; one wave per row spent
+// its time in the six steps of its sum and waited for two loads at a time.
+// Diffusion 48^3 p = 2 FP64 (14.5 M entries, resident in the last level cache):
+// 29.3 -> 20 us, of which the shapes' 8 B per entry instead of 12 give a third.
+template <typename V, typename ACC, bool DOT, bool SKIP, typename VV, bool SHAPED, int L, int U>
 __global__ __launch_bounds__(kThreads) void k_spmv_dot(
     int n, const int64_t* __restrict__ rowptr, const int32_t* __restrict__ start,
     const int32_t* __restrict__ cols, const VV* __restrict__ val, const V* __restrict__ p,
@@ -56,14 +56,14 @@ __global__ __launch_bounds__(kThreads) void k_spmv_dot(
 {
   if (SKIP && scal[S_DONE] != 0.0) return;
   __shared__ double sh[kThreads / 64];
-  constexpr int L = kRowLanes, groups = kThreads / L;
+  constexpr int groups = kThreads / L;
   const int g = threadIdx.x / L, l = threadIdx.x % L;
   double pq = 0.0;
   for (int row = blockIdx.x * groups + g; row < n; row += gridDim.x * groups) {
     const int64_t b = rowptr[row];
     const int cnt = (int)(rowptr[row + 1] - b);
-    ACC s = group_sum<L>(row_dot<L, ACC>(l, cnt, val + b, SHAPED ? cols + start[row] : cols + b,
-                                         SHAPED ? p + row : p));
+    ACC s = group_sum<L>(row_dot<L, U, ACC>(l, cnt, val + b, SHAPED ? cols + start[row] : cols + b,
+                                            SHAPED ? p + row : p));
     if (!std::is_same<VV, V>::value) s *= scale;
     if (l == 0) {
       q[row] = (V)s;
@@ -77,16 +77,15 @@ __global__ __launch_bounds__(kThreads) void k_spmv_dot(
 
 // SpMV for 3-component systems whose DOFs are free or fixed per node: the
 // three rows of a node share one column pattern made of node triples, so the
-// gather reads one node index (bcol) per 9 values.  16 lanes per node; the
-// CSR values are read in place.  Blocks are mapped to the 8 XCDs in
+// gather reads one node index (bcol) per 9 values.  L lanes per node, U
+// neighbours each in a round; the CSR values are read in place.  Blocks are mapped to the 8 XCDs in
 // contiguous node ranges so each XCD's L2 holds its slice of p.
 // SHAPED: node columns from the row shapes (start per node, table `cols`).
 // Bound by the reading of the values.  Elasticity 64^3 p = 2 FP64 (2.4 GB):
 // 524 us with one wave per node and column indices, 494 with row shapes, 427
 // (5.7 TB/s) with 16 lanes and four neighbours ahead per lane; 439 with 8
-// lanes, 455 with 32 and two ahead.
-template <typename V, typename ACC, bool DOT, bool SKIP = DOT, typename VV = V,
-          bool SHAPED = false>
+// lanes, 443 with 32, 455 with 32 and two ahead.
+template <typename V, typename ACC, bool DOT, bool SKIP, typename VV, bool SHAPED, int L, int U>
 __global__ __launch_bounds__(kThreads) void k_spmv_node3(
     int nnode, const int64_t* __restrict__ rowptr, const int32_t* __restrict__ start,
     const int32_t* __restrict__ cols, const VV* __restrict__ val, const V* __restrict__ p,
@@ -94,7 +93,7 @@ __global__ __launch_bounds__(kThreads) void k_spmv_node3(
 {
   if (SKIP && scal[S_DONE] != 0.0) return;
   __shared__ double sh[kThreads / 64];
-  constexpr int L = kNodeLanes, GPB = kThreads / L;
+  constexpr int GPB = kThreads / L;
   const int g = threadIdx.x / L, lane = threadIdx.x % L;
   const int nxcd = 8;
   const int xcd = blockIdx.x % nxcd, bl = blockIdx.x / nxcd, nbl = gridDim.x / nxcd;
@@ -104,8 +103,8 @@ __global__ __launch_bounds__(kThreads) void k_spmv_node3(
     const int64_t r0 = rowptr[3 * nd];
     const int cnt = (int)((rowptr[3 * nd + 1] - r0) / 3);
     ACC t[3];
-    node_dots<L>(lane, cnt, val + r0, SHAPED ? cols + start[nd] : cols + r0 / 9,
-                     SHAPED ? p + 3 * (int64_t)nd : p, t);
+    node_dots<L, U>(lane, cnt, val + r0, SHAPED ? cols + start[nd] : cols + r0 / 9,
+                    SHAPED ? p + 3 * (int64_t)nd : p, t);
     ACC s0 = group_sum<L>(t[0]), s1 = group_sum<L>(t[1]), s2 = group_sum<L>(t[2]);
     if (!std::is_same<VV, V>::value) {
       s0 *= scale;
@@ -409,6 +408,32 @@ __global__ void k_demote_scaled(int n, const double* __restrict__ r, float* __re
 }
 
 // ---------------------------------------------------------------------------
+// Lanes of a product per row, or per node: few where a round of them covers a
+// list (linear elements), many where the rows are too few to fill the chip and
+// a list would take many rounds one after the other.
+//   rows of at most 40 entries: 4 lanes of four pairs.  Linear scalar elements
+//   90^3: 36 us, 62 with 8 lanes, FP32 25 and 49.
+//   long rows of small systems: 32 lanes of two pairs.  Cubic scalar 8^3 3.4
+//   us, 5.0 with 8 lanes; at 28^3 (24k rows) 8 lanes are as fast, FP32 faster.
+//   nodes of at most 32 neighbours (linear elements): 16 lanes.
+//   long lists of few nodes: 64 lanes of two.  Cubic elasticity 8^3 5.4 us, 8.4
+//   with 16 lanes, 5.5 with 32; from 30^3 (35k nodes) on 32 lanes read faster.
+//   others: 32 lanes (quadratic 24^3 21.5 us, 23.7 with 16), but 16 for FP64
+//   values that come from HBM (quadratic 64^3 429 us, 443 with 32).
+template <typename V>
+static int product_lanes(const Context& c)
+{
+  if (!c.d_bcol) {
+    const double len = c.neq > 0 ? (double)c.nnz / c.neq : 0.0;
+    return len <= 40 ? 4 : len > 120 && c.neq <= 16384 ? 32 : 8;
+  }
+  const int nodes = c.neq / 3;
+  const double len = nodes > 0 ? (double)c.nnz / 9 / nodes : 0.0;
+  if (len <= 32) return 16;
+  if (len > 128) return nodes <= 16384 ? 64 : 32;
+  return sizeof(V) == 8 && nodes > 131072 ? 16 : 32;
+}
+
 // Blocks of a product (a multiple of the 8 XCDs): one pass over the rows where
 // that takes few, else 4 per CU, 8 for FP64 node triples.  4 leave the CUs
 // evenly loaded and half the partials to add up: mixed elasticity step 40^3
@@ -418,7 +443,7 @@ __global__ void k_demote_scaled(int n, const double* __restrict__ r, float* __re
 template <typename V>
 static int spmv_grid(const Context& c)
 {
-  const int rows = c.d_bcol ? c.neq / 3 : c.neq, per = kThreads / (c.d_bcol ? kNodeLanes : kRowLanes);
+  const int rows = c.d_bcol ? c.neq / 3 : c.neq, per = kThreads / product_lanes<V>(c);
   const int need = (rows + per - 1) / per, cap = c.d_bcol && sizeof(V) == 8 ? kGrid : kGrid / 2;
   return need < cap ? (need + 7) / 8 * 8 : cap;
 }
@@ -442,14 +467,23 @@ static void launch_spmv(Context& c, const VV* val, const V* p, V* q, ACC scale =
     kernel<<<grid, kThreads, 0, st>>>(n, c.d_rowptr, start, cols, val, p, q, w.partial, w.scal,
                                        scale);
   };
-  if (c.d_bcol && sh.start)
-    run(k_spmv_node3<V, ACC, DOT, SKIP, VV, true>, c.neq / 3, sh.start, sh.table);
-  else if (c.d_bcol)
-    run(k_spmv_node3<V, ACC, DOT, SKIP, VV>, c.neq / 3, nullptr, c.d_bcol);
-  else if (sh.start)
-    run(k_spmv_dot<V, ACC, DOT, SKIP, VV, true>, c.neq, sh.start, sh.table);
+  const int lanes = product_lanes<V>(c);
+  auto rows = [&](auto shaped, const int32_t* start, const int32_t* cols) {
+    constexpr bool S = decltype(shaped)::value;
+    if (lanes == 4) run(k_spmv_dot<V, ACC, DOT, SKIP, VV, S, 4, 4>, c.neq, start, cols);
+    else if (lanes == 8) run(k_spmv_dot<V, ACC, DOT, SKIP, VV, S, 8, 4>, c.neq, start, cols);
+    else run(k_spmv_dot<V, ACC, DOT, SKIP, VV, S, 32, 2>, c.neq, start, cols);
+  };
+  auto nodes = [&](auto shaped, const int32_t* start, const int32_t* cols) {
+    constexpr bool S = decltype(shaped)::value;
+    if (lanes == 16) run(k_spmv_node3<V, ACC, DOT, SKIP, VV, S, 16, 4>, c.neq / 3, start, cols);
+    else if (lanes == 32) run(k_spmv_node3<V, ACC, DOT, SKIP, VV, S, 32, 4>, c.neq / 3, start, cols);
+    else run(k_spmv_node3<V, ACC, DOT, SKIP, VV, S, 64, 2>, c.neq / 3, start, cols);
+  };
+  if (c.d_bcol)
+    sh.start ? nodes(std::true_type(), sh.start, sh.table) : nodes(std::false_type(), nullptr, c.d_bcol);
   else
-    run(k_spmv_dot<V, ACC, DOT, SKIP, VV>, c.neq, nullptr, c.d_colind);
+    sh.start ? rows(std::true_type(), sh.start, sh.table) : rows(std::false_type(), nullptr, c.d_colind);
 }
 
 // FP32 SpMV for the multigrid smoother on the finest level.

@@ -14,16 +14,16 @@ struct Pack {
 };
 
 // Row sum: entries m < cnt of v times x at columns ci[m].  The entries go out
-// in pairs, a sum for each half; U pairs per lane are requested before the
-// first is used (past the end the last pair once more, its products dropped;
+// in pairs, a sum for each half; U pairs per lane (2 L U entries of a row in a
+// round) are requested before the first is used (past the end the last pair once more, its products dropped;
 // left to the compiler the loads of x go out between the products, and the
 // batch of k_bspmv takes 72 instead of 61 ms).  Rows start at any entry, so
 // the pairs are aligned to one entry only.
-template <int L, typename ACC, typename VV, typename V>
+template <int L, int U, typename ACC, typename VV, typename V>
 __device__ inline ACC row_dot(int l, int cnt, const VV* __restrict__ v,
                               const int32_t* __restrict__ ci, const V* __restrict__ x)
 {
-  constexpr int W = 2, U = 4;
+  constexpr int W = 2;
   ACC s[W] = {};
   const int nv = cnt / W;
   for (int k0 = 0; k0 < nv; k0 += L * U) {
@@ -58,13 +58,12 @@ __device__ inline ACC row_dot(int l, int cnt, const VV* __restrict__ v,
 }
 
 // The three row sums of a node: cnt neighbour nodes ci[k], whose three values
-// per row are consecutive (rows 3 cnt apart).
-template <int L, typename ACC, typename VV, typename V>
+// per row are consecutive (rows 3 cnt apart); U neighbours per lane in a round.
+template <int L, int U, typename ACC, typename VV, typename V>
 __device__ inline void node_dots(int l, int cnt, const VV* __restrict__ v,
                                  const int32_t* __restrict__ ci, const V* __restrict__ x,
                                  ACC (&s)[3])
 {
-  constexpr int U = 4;
   s[0] = s[1] = s[2] = 0;
   for (int k0 = 0; k0 < cnt; k0 += L * U) {
     Pack<VV, 3> a[U][3];

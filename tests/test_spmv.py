@@ -1,7 +1,8 @@
 """Matrix-vector products (GPU) over the row layouts they tell apart: scalar
-rows and node triples, columns from row shapes (free or face-fixed patches) and
-from the column indices (fixings strewn over the patch), rows shorter and
-longer than a group's stride, one and several groups per row list.
+rows and node triples, columns from row shapes (free or face-fixed patches that
+are large enough for their lists to repeat) and from the column indices (small
+patches, fixings strewn over the patch), rows shorter and longer than a round
+of their lanes, each number of lanes.
 
 A sum of n products is within n units of roundoff of its exact value, relative
 to the sum of the absolute products; rows hold at most 1029 entries and both
@@ -42,6 +43,49 @@ def test_product_of_every_row_layout(nc, p, nel, fix):
     else:
         itg = M.Integrand(M.POISSON, source=M.smooth_source(4, 4))
     print(f"[gpu] spmv nc={nc} p={p} nel={nel} fix={fix} neq={neq}", flush=True)
+    _check_products(P, itg, nc, p, meqn, neq)
+
+
+def _shapes_kept(rp, ci, nodal):
+    """Whether the distinct lists of column offsets take at most an eighth of
+    the (node) column indices: the products then read the lists."""
+    if nodal:
+        n = (len(rp) - 1) // 3
+        cnt = np.diff(rp)[::3] // 3
+        start = np.concatenate([[0], np.cumsum(cnt)])
+        ci = np.concatenate([ci[rp[3 * k]:rp[3 * k + 1]:3] // 3 for k in range(n)])
+    else:
+        n, start = len(rp) - 1, rp
+    lists = {(ci[start[r]:start[r + 1]] - r).tobytes() for r in range(n)}
+    return sum(map(len, lists)) // ci.itemsize <= start[-1] // 8
+
+
+# lanes: of the rows or nodes of this size (4 or 16: short lists; 32 or 64: long
+# lists of few rows; 8 or 32: others)
+@pytest.mark.parametrize("nc,p,nel,lanes", [
+    (1, 1, (16, 9, 8), 4), (1, 2, (12, 10, 11), 8), (1, 3, (12, 11, 13), 32),
+    (1, 3, (30, 26, 24), 8), (3, 1, (14, 9, 8), 16), (3, 2, (12, 10, 11), 32),
+    (3, 3, (13, 11, 12), 64), (3, 3, (150, 20, 2), 32)])
+def test_products_from_row_shapes(nc, p, nel, lanes):
+    P = M.cube_patch(p, list(nel), 0.1, seed=p + nc)
+    fix = [7, 0, 0, 7, 0, 0] if nc == 3 else [0] * 6
+    meqn, neq = M.equation_numbers(M.face_status(P, nc, fix))
+    if nc == 3:
+        itg = M.Integrand(M.ELASTICITY, E=1.3, nu=0.28, body=(0.2, -0.1, 0.3))
+    else:
+        itg = M.Integrand(M.POISSON, source=M.smooth_source(4, 4))
+    print(f"[gpu] spmv shapes nc={nc} p={p} nel={nel} neq={neq}", flush=True)
+    rp, ci = _check_products(P, itg, nc, p, meqn, neq)
+    assert _shapes_kept(rp, ci, nc == 3)
+    length = len(ci) / neq / nc
+    if nc == 1:
+        want = 4 if length <= 40 else 32 if length > 120 and neq <= 16384 else 8
+    else:
+        want = 16 if length <= 32 else 64 if length > 128 and neq <= 3 * 16384 else 32
+    assert want == lanes
+
+
+def _check_products(P, itg, nc, p, meqn, neq):
     x = np.random.default_rng(neq).standard_normal(neq)
     hole = neq // 2
     xi = x.copy()
@@ -71,3 +115,4 @@ def test_product_of_every_row_layout(nc, p, nel, fix):
     rows[np.repeat(np.arange(neq), np.diff(rp))[ci == hole]] = True
     assert np.array_equal(np.isfinite(yi), ~rows)
     assert np.array_equal(yi[~rows], y[~rows])
+    return rp, ci
