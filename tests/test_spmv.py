@@ -7,13 +7,16 @@ of their lanes, each number of lanes.
 A sum of n products is within n units of roundoff of its exact value, relative
 to the sum of the absolute products; rows hold at most 1029 entries and both
 sides round: 2.3e-13 (FP64), 6.2e-5 (FP32 against an FP64 sum)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import scipy.sparse as sp
 import torch
 
-from ifem_amd import FP32, FP64, Session
+from ifem_amd import FP32, FP64, Session, lib
 from ifem_amd import model as M
+from ifem_amd._native import check
 
 pytestmark = pytest.mark.gpu
 
@@ -116,3 +119,64 @@ def _check_products(P, itg, nc, p, meqn, neq):
     assert np.array_equal(np.isfinite(yi), ~rows)
     assert np.array_equal(yi[~rows], y[~rows])
     return rp, ci
+
+
+def _hip(name, *args):
+    """A call of the HIP runtime that the library is linked with."""
+    rc = getattr(lib(), name)(*args)
+    assert rc == 0, (name, rc)
+
+
+def test_row_shapes_come_with_the_first_product():
+    """The search for row shapes is the first product's, not the set-up's, so
+    every way to make that product has to give the same bits: recorded in a
+    graph (no search can be made there), without allocation, plain, and after a
+    system of another pattern in the same session."""
+    def bind(s, nel, p):
+        P = M.cube_patch(p, list(nel), 0.1, seed=p)
+        meqn, neq = M.equation_numbers(M.face_status(P, 1, [0] * 6))
+        s.bind(s.add_patch(P), 1, meqn, neq)
+        s.init_assembly()
+        s.assemble(M.Integrand(M.POISSON, source=M.smooth_source(4, 4)), (p + 1,) * 3, FP64)
+        return neq
+
+    def noalloc(s, x):
+        y = np.empty_like(x)
+        check(lib().ifem_gpu_spmv_noalloc(s.h, x.ctypes.data_as(C.c_void_p), y.ctypes.data_as(C.c_void_p)))
+        return y
+    nel = (16, 14, 12)
+    print("[gpu] spmv first products", flush=True)
+    with Session() as s:
+        neq = bind(s, nel, 2)
+        x = np.random.default_rng(neq).standard_normal(neq)
+        plain = s.spmv(x)
+        assert np.array_equal(noalloc(s, x), plain)
+        n2 = bind(s, (9, 20, 11), 1)  # another pattern, shapes of the first one held
+        rp, ci, A, _ = s.system()
+        x2 = np.random.default_rng(n2).standard_normal(n2)
+        K = sp.csr_matrix((A, ci, rp), shape=(n2, n2))
+        assert np.all(np.abs(s.spmv(x2) - K @ x2) <= 2.3e-13 * (abs(K) @ np.abs(x2)))
+    with Session() as s:
+        bind(s, nel, 2)
+        assert np.array_equal(noalloc(s, x), plain)
+        assert np.array_equal(s.spmv(x), plain)
+    with Session() as s:
+        bind(s, nel, 2)
+        xd = torch.from_numpy(x).cuda()
+        yd = torch.zeros_like(xd)
+        torch.cuda.synchronize()
+        stream, graph, run = C.c_void_p(s.stream), C.c_void_p(), C.c_void_p()
+        s.synchronize()
+        _hip("hipStreamBeginCapture", stream, C.c_int(0))  # global: no allocation meanwhile
+        s.spmv_device(xd.data_ptr(), yd.data_ptr())
+        _hip("hipStreamEndCapture", stream, C.byref(graph))
+        _hip("hipGraphInstantiate", C.byref(run), graph, None, None, C.c_size_t(0))
+        for scale in (1.0, 2.0, -1.0):
+            xd.copy_(torch.from_numpy(scale * x))
+            torch.cuda.synchronize()
+            _hip("hipGraphLaunch", run, stream)
+            s.synchronize()
+            assert np.array_equal(yd.cpu().numpy(), scale * plain)
+            assert np.array_equal(s.spmv(x), plain)
+        _hip("hipGraphExecDestroy", run)
+        _hip("hipGraphDestroy", graph)
