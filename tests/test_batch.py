@@ -119,6 +119,43 @@ def test_batch_mixed_precision_and_autotune():
             assert np.linalg.norm(b - K @ x) <= 1e-8 * np.linalg.norm(b) * 1.01, k
 
 
+def test_batch_with_row_shapes_and_row_segments():
+    """Patches large enough for the product to read row shapes (distinct lists
+    of column offsets at most an eighth of all; the small batches above read
+    column indices) and few enough for lines to be cut into row segments: K and
+    b against the oracle, solutions by the host's residual and energy norm."""
+    pbs = problems.diffusion_batch(6, (12, 16), (1, 2, 3), sigma=1.0, ell=0.2, seed=9, nmodes=32)
+    degrees = [pb.patch.p[0] for pb in pbs]
+    _say(f"[gpu] batch with row shapes, p={degrees}")
+    assert set(degrees) == {1, 2, 3}
+    with setup_batch(pbs, precisions=(FP64, FP32)) as s:
+        K, lists, entries = [], 0, 0
+        for k, pb in enumerate(pbs):
+            rp, ci, A, b = _oracle(pb)
+            grp, gci, gA, gA32, gb = s.batch_system(k, values32=True)
+            assert np.array_equal(grp, rp) and np.array_equal(gci, ci), k
+            assert np.max(np.abs(gA - A)) <= 1e-12 * np.max(np.abs(A)), k
+            assert np.max(np.abs(gb - b)) <= 1e-12 * np.max(np.abs(b)), k
+            assert np.max(np.abs(gA32 - A)) <= 1e-5 * np.max(np.abs(A)), k
+            K.append((sp.csr_matrix((gA, gci, grp), shape=(pb.neq, pb.neq)), gb))
+            lists += sum({(ci[rp[r]:rp[r + 1]] - r).tobytes(): rp[r + 1] - rp[r]
+                          for r in range(pb.neq)}.values())
+            entries += len(ci)
+        assert lists <= entries // 8
+        st = s.batch_solve(rtol=1e-12, maxits=5000)
+        x64 = [s.batch_solution(k) for k in range(len(pbs))]
+        assert st["converged"]
+        for k, (A, b) in enumerate(K):
+            assert np.linalg.norm(b - A @ x64[k]) <= 1e-12 * np.linalg.norm(b) * 1.01, k
+        st = s.batch_solve(rtol=1e-8, maxits=5000, precision=FP32, inner_rtol=1e-4)
+        assert st["converged"]
+        for k, (A, b) in enumerate(K):
+            x = s.batch_solution(k)
+            e = x - x64[k]
+            assert np.sqrt(e @ (A @ e)) <= 1e-6 * np.sqrt(x64[k] @ (A @ x64[k])), k
+            assert np.linalg.norm(b - A @ x) <= 1e-8 * np.linalg.norm(b) * 1.01, k
+
+
 def test_batch_errors():
     from ifem_amd import GpuError, Session
     from ifem_amd import model as M
@@ -170,7 +207,7 @@ def test_batch_full_size_properties():
         assert np.max(np.abs(gb - b)) <= 1e-12 * np.max(np.abs(b))
         # a mid-size p = 3 block against the oracle (full bundles, many work
         # items per workgroup), and every block's FP32 values against its FP64
-        # ones (the two precisions run different kernels)
+        # ones (instances of their own)
         mid = [(pb.neq, q) for q, pb in enumerate(pbs)
                if pb.patch.p[0] == 3 and min(np.array(pb.patch.n) - 3) >= 12]
         k = min(mid)[1]
