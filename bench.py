@@ -54,6 +54,21 @@ def measured_traffic(kernel):
     return None
 
 
+def line_kernel(pb):
+    """(name, operations) of the FP64 line kernel of a one-patch quadratic
+    elasticity problem without body force: the operations that the sum
+    factorisation (csrc/lines.hpp) makes on lines that are not split.  Per line
+    and element layer: units (9 component pairs x 9 derivative pairs x ng points)
+    over the element rows that touch the line, then column lines; the Lame
+    combinations per entry."""
+    p, ng, (n1, n2, n3), (m1, _, m3) = pb.patch.p[0], pb.ng[0], pb.patch.n, pb.patch.nel
+    P1, W1, q = p + 1, 2 * p + 1, (p + 1) * ng
+    units = n2 * m1 * (P1 * m3) * (ng * 81) * ng * (q * (1 + 2 * P1) + 2 * P1 * W1)
+    columns = n2 * n3 * m1 * (9 * W1 * W1) * ng * (5 + 6 * P1 + 4 * P1 * P1)
+    rows = n1 * n2 * n3 * 9 * W1 ** 3 * 4
+    return f"k_lines<{p}, {ng}, 3, double, false, false, false>", float(units + columns + rows)
+
+
 def _train_net(LN, Session, spec, X, T, epochs, lr=1e-3):
     """Adam in three stages of halving learning rate; returns (params,
     target scale, loss first/last, seconds)."""
@@ -453,8 +468,6 @@ def main():
     pb = problems.elasticity_cube(args.nel, 2)
     ndof, neq = pb.ndof, pb.neq
     nel_tot = int(np.prod(pb.patch.nel))
-    nen = pb.patch.nen
-    ngp = int(np.prod(pb.ng))
     log(f"[bench] workload elasticity {args.nel}^3 p=2: ndof={ndof} neq={neq}")
 
     s = Session(stream=stream.cuda_stream)
@@ -515,9 +528,9 @@ def main():
         e1.record(stream)
     stream.synchronize()
     spmv_ms = e0.elapsed_time(e1) / args.spmv_reps
-    # node-triple index: values + one int32 per 9 values + 2 row pointers per
-    # node + x read + y written (3-component node-uniform system)
-    spmv_bytes = nnz * 8 + (nnz // 9) * 4 + (neq // 3) * 2 * 8 + 2 * neq * 8
+    # node triples with row shapes: values + a shape start and 2 row pointers
+    # per node + x read + y written (3-component node-uniform system)
+    spmv_bytes = nnz * 8 + (neq // 3) * (4 + 2 * 8) + 2 * neq * 8
 
     if args.copy_calibration:
         copy_calibration(stream)
@@ -690,14 +703,14 @@ def main():
         log(f"[bench] cpu baseline: {cpu}")
 
     # ---- roofline of the dominant assembly kernel -------------------------------
-    flops = (36 * nen * nen + 6 * nen) * ngp * nel_tot
+    kname, flops = line_kernel(pb)
     asm_bytes = nnz * 8 + neq * 8 + pb.patch.nnod * 3 * 8
     achieved = flops / (lines_ms * 1e-3)
-    traffic = measured_traffic("ifem::k_assemble_lines<2, 3, 3, double, 1, false, 0>") \
-        if args.nel == 64 else None
-    # compute-bound: FP64 FMAs on the vector ALUs (MI355X's FP64 vector and
-    # FP64 matrix peaks are the same 78.6 TFLOP/s)
-    roofline = {"kernel": "k_assemble_lines<2,3,3,double,1,false,0>", "bound": "mfma",
+    traffic = measured_traffic("ifem::" + kname) if args.nel == 64 else None
+    # FP64 FMAs on the vector ALUs (MI355X's FP64 vector and FP64 matrix peaks
+    # are the same 78.6 TFLOP/s); the kernel waits on LDS and between its
+    # barriers for most of the time
+    roofline = {"kernel": kname.replace(" ", ""), "bound": "latency",
                 "engine": "valu_fp64",
                 "achieved": round(achieved / 1e12, 3), "peak": PEAK_FP64 / 1e12,
                 "unit": "TFLOP/s", "frac": round(achieved / PEAK_FP64, 4), "traffic": traffic,
@@ -707,11 +720,13 @@ def main():
                                    "max_roofline_frac": round(max(flops / PEAK_FP64,
                                                                   asm_bytes / PEAK_HBM)
                                                               / (kern_ms * 1e-3), 4)}}
-    spmv_roof = {"kernel": "k_spmv_node3<double,double,false,false,double>", "bound": "hbm",
+    lanes = 16 if neq // 3 > 131072 else 32
+    sname = f"k_spmv_node3<double, double, false, false, double, true, {lanes}, 4>"
+    spmv_roof = {"kernel": sname.replace(" ", ""), "bound": "hbm",
                  "achieved": round(spmv_bytes / (spmv_ms * 1e-3) / 1e9, 1), "peak": 8000.0,
                  "unit": "GB/s", "frac": round(spmv_bytes / (spmv_ms * 1e-3) / PEAK_HBM, 4),
-                 "traffic": (measured_traffic("ifem::k_spmv_node3<double, double, false, false, double>")
-                             if args.nel == 64 else None), "bytes": spmv_bytes, "kernel_ms": round(spmv_ms, 4)}
+                 "traffic": measured_traffic("ifem::" + sname) if args.nel == 64 else None,
+                 "bytes": spmv_bytes, "kernel_ms": round(spmv_ms, 4)}
 
     value = ndof / (asm_ms * 1e-3)
     out = {
