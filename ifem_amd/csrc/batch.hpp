@@ -35,8 +35,9 @@ struct RowShapes {
   void release();
 };
 
-// Per-degree tuning: work list of the assembly (half: segments of half the
-// length) and row entries per step of the SpMV.
+// Per-degree tuning: work split of the assembly (half: row segments of half the
+// length at degrees 1 and 2, half element chunks at degree 3) and row entries
+// per step of the SpMV.
 struct BatchTune {
   int half = 0;
   int lanes = 0; // 0: the default

@@ -180,8 +180,8 @@ struct Context {
   void* d_asmargs = nullptr; // assembly kernel arguments (device copy)
   double* d_gpgeo = nullptr; // geometry records per (element, Gauss point)
   size_t gpgeo_cap = 0;      // doubles
-  // element-chunk variant of the line kernel per (p, ng-p-1, ncomp==3, fp32):
-  // -1 built-in default, 0 full, 1 half
+  // work split of the line kernel per (p, ng-p-1, ncomp==3, fp32), as
+  // ifem_gpu_set_assembly_variant takes it: -1 the built-in choice
   int asm_half[4][2][2][2] = {{{{-1, -1}, {-1, -1}}, {{-1, -1}, {-1, -1}}},
                               {{{-1, -1}, {-1, -1}}, {{-1, -1}, {-1, -1}}},
                               {{{-1, -1}, {-1, -1}}, {{-1, -1}, {-1, -1}}},

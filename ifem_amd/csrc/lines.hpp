@@ -26,12 +26,12 @@
 // component pair, and the sum over the layer's elements needs no reduction.
 // Bound: the units read two LDS values per four FP64 operations (one in
 // scalar problems), which makes LDS bandwidth and FP64 issue about equal (34 %
-// and 37 % of the time at 64^3 p = 2 elasticity, two waves per SIMD); the rest
+// and 38 % of the time at 64^3 p = 2 elasticity, two waves per SIMD); the rest
 // is latency between the barriers.  Against direct quadrature with one line
 // per workgroup (lines_direct.hpp): 64^3 p = 2 elasticity 6.39 -> 4.15 ms, two
 // 16x32x32 patches 0.89 -> 0.65 ms each, 45x37x51 p = 2 Poisson 1.12 -> 0.26 ms.
-// Each XCD runs a contiguous range of groups: the records are fetched 0.97 GB
-// instead of 5 GB at 64^3 elasticity.
+// Each XCD runs a contiguous range of groups: 2.0 GB are fetched instead of 4.9
+// at 64^3 elasticity (the records are 0.57 GB).
 // Every K entry is written once, without atomics, and all sums have a fixed
 // order that does not depend on how the rows are split into workgroups, so
 // results are bitwise reproducible.

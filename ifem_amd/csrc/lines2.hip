@@ -10,8 +10,10 @@ int launch_lines2(Context& c, const AsmArgs& a, int ng, bool fp32, bool rhs, int
   // FP32 elasticity stays with the direct kernel: the sum-factorised FP32
   // matrix is closer to the FP64 one (4.5e-8 against 7.4e-8 relative), but
   // the mixed-precision solve, whose time it is made for, then needs 7 %
-  // more inner iterations (718 against 671 on 40^3 elasticity, mean of 12
-  // systems)
+  // more inner iterations: 718 against 671 on 40^3 elasticity, 465 against 432
+  // on 24^3, means of 12 systems.  Both errors are far below the inner
+  // tolerance of 1e-4, and why the rounding tells is not known; 7 % of a
+  // solve is more than the whole FP32 assembly takes (64^3 4.4 ms)
   if (fp32 && c.ncomp == 3) {
     launch_direct_v<2, 3, 3, float>(c, a, false, variant);
     IFEM_HIP(hipGetLastError());

@@ -427,6 +427,7 @@ __device__ __forceinline__ void line_impl(
 #pragma unroll
         for (int s = 0; s < NS; s++) acc[a1][s] = 0;
         if constexpr (PIPE) {
+        static_assert(NC == 3 && !HAS_RHS, "FP32 elasticity with 3x3x3 points");
         const int m2 = e2 - jc + P, m3 = e3 - kc + P;
         T vn1[NG], vd1[NG], vn2[NG], vd2[NG], vn3[NG], vd3[NG];
 #pragma unroll
@@ -465,29 +466,23 @@ __device__ __forceinline__ void line_impl(
           const T n23 = vn2[q2] * vn3[q3], d23 = vd2[q2] * vn3[q3], n2d3 = vn2[q2] * vd3[q3];
           const T r0 = vd1[q1] * n23, r1 = vn1[q1] * d23, r2 = vn1[q1] * n2d3;
           const T* G = PREF ? Gc : Gbase + qq * LL::GEO;
-          if (NC == 1) {
+          const T gb0 = r0 * G[0] + r1 * G[3] + r2 * G[6];
+          const T gb1 = r0 * G[1] + r1 * G[4] + r2 * G[7];
+          const T gb2 = r0 * G[2] + r1 * G[5] + r2 * G[8];
 #pragma unroll
-            for (int a1 = 0; a1 < P1; a1++)
-              acc[a1][0] += r0 * G[3 * a1] + r1 * G[3 * a1 + 1] + r2 * G[3 * a1 + 2];
-          } else {
-            const T gb0 = r0 * G[0] + r1 * G[3] + r2 * G[6];
-            const T gb1 = r0 * G[1] + r1 * G[4] + r2 * G[7];
-            const T gb2 = r0 * G[2] + r1 * G[5] + r2 * G[8];
+          for (int a1 = 0; a1 < P1; a1++) {
+            const T wa0 = G[9 + 3 * a1], wa1 = G[10 + 3 * a1], wa2 = G[11 + 3 * a1];
+            if constexpr (SACC) {
+              acc[a1][0] += wa0 * gb0; acc[a1][1] += wa0 * gb1; acc[a1][2] += wa0 * gb2;
+              acc[a1][3] += wa1 * gb0; acc[a1][4] += wa1 * gb1; acc[a1][5] += wa1 * gb2;
+              acc[a1][6] += wa2 * gb0; acc[a1][7] += wa2 * gb1; acc[a1][8] += wa2 * gb2;
+            } else {
+              const T wa[3] = {wa0, wa1, wa2}, gb[3] = {gb0, gb1, gb2};
+              const T dot = wa0 * gb0 + wa1 * gb1 + wa2 * gb2;
 #pragma unroll
-            for (int a1 = 0; a1 < P1; a1++) {
-              const T wa0 = G[9 + 3 * a1], wa1 = G[10 + 3 * a1], wa2 = G[11 + 3 * a1];
-              if constexpr (SACC) {
-                acc[a1][0] += wa0 * gb0; acc[a1][1] += wa0 * gb1; acc[a1][2] += wa0 * gb2;
-                acc[a1][3] += wa1 * gb0; acc[a1][4] += wa1 * gb1; acc[a1][5] += wa1 * gb2;
-                acc[a1][6] += wa2 * gb0; acc[a1][7] += wa2 * gb1; acc[a1][8] += wa2 * gb2;
-              } else {
-                const T wa[3] = {wa0, wa1, wa2}, gb[3] = {gb0, gb1, gb2};
-                const T dot = wa0 * gb0 + wa1 * gb1 + wa2 * gb2;
-#pragma unroll
-                for (int jj = 0; jj < 3; jj++)
-                  acc[a1][jj] += lam * wa[rc] * gb[jj] + mu * wa[jj] * gb[rc] +
-                                 (jj == rc ? mu * dot : T(0));
-              }
+              for (int jj = 0; jj < 3; jj++)
+                acc[a1][jj] += lam * wa[rc] * gb[jj] + mu * wa[jj] * gb[rc] +
+                               (jj == rc ? mu * dot : T(0));
             }
           }
           if (PREF && qq + 1 < ngs) {
@@ -504,7 +499,6 @@ __device__ __forceinline__ void line_impl(
           __syncthreads();
           phase_a(qa1, ngs1);
           __syncthreads();
-          if (HAS_RHS) rhs_reduce(ngs1);
           slab_b(std::integral_constant<int, 1>{});
         }
         } else if constexpr (LL::SF) {
@@ -1090,15 +1084,14 @@ __global__ __launch_bounds__(kBlock, HALF == 2 ? 3 : 1) void k_assemble_lines(
                                                       be2, be3, eqw, pbase, prow, &nbundle);
 }
 
-// Persistent batch assembly over many independent patches, one launch per
-// degree p = 1..3 (ng = p+1) present in the batch, each with the single-patch
-// kernel's own phase-B and window-update variants and its own register and
-// LDS budget.  Work items are (patch, line) pairs sorted by decreasing cost
-// within the degree; blocks take the next item from the degree's queue
-// counter, so load balances over patches of uneven size.  Each line's rows
-// are written by exactly one block, so the result does not depend on which
-// block takes which item.  HALF: the element-chunk variant chosen for the
-// degree (AsmArgs::variant = 2*(p-1) + HALF for every patch of it).
+// Persistent batch assembly of a batch's patches of degree 3 (ng = 4; degrees
+// 1 and 2: k_lines_batch), with the single-patch kernel's own phase-B and
+// window-update variants and its own register and LDS budget.  Work items are
+// whole lines of a patch sorted by decreasing cost; blocks take the next item
+// from the degree's queue counter, so load balances over patches of uneven
+// size.  Each line's rows are written by exactly one block, so the result does
+// not depend on which block takes which item.  HALF: the element-chunk variant
+// (BatchTune::half).
 template <int P, typename T, bool HAS_RHS, int HALF>
 __global__ __launch_bounds__(kBlock, 3) void k_assemble_batch(const AsmArgs* __restrict__ args,
                                                            const LineItem* __restrict__ items,

@@ -8,7 +8,7 @@
 namespace ifem {
 
 // Rows of the bound patch: variant 0 splits the lines into row segments by
-// the rule in launch_lines_t, 1 into twice as many, 2 not at all.
+// the rule in row_segments, 1 into twice as many, 2 not at all.
 int launch_lines1(Context& c, const AsmArgs& args, int ng, bool fp32, bool rhs, int variant);
 int launch_lines2(Context& c, const AsmArgs& args, int ng, bool fp32, bool rhs, int variant);
 int launch_lines3(Context& c, const AsmArgs& args, int ng, bool fp32, bool rhs, int variant);

@@ -376,8 +376,8 @@ int ifem_gpu_mg_apply(ifem_gpu_ctx* ctx, const double* r, double* z);
 
 /* ---- batch of independent patches ------------------------------------------
  * Many scalar (Poisson / diffusion) patches, each with its own SAM numbering
- * and integrand, assembled by one persistent launch into one block-diagonal
- * system and solved together with one Jacobi-PCG per patch (own scalars and
+ * and integrand, assembled by one persistent launch per degree into one
+ * block-diagonal system and solved together with one Jacobi-PCG per patch (own scalars and
  * convergence test; the iteration loop is replayed from a captured hipGraph).
  * Per patch, assembly and solve are those of ifem_gpu_assemble and
  * ifem_gpu_solve; the batch stands in for the per-patch loop of
@@ -396,12 +396,14 @@ int ifem_gpu_batch_add(ifem_gpu_ctx* ctx, int patch_id, const int* meqn, int neq
  * patch, src/LinAlg/SparseMatrix.C:717-762), work list and solver buffers.
  * neq, nnz (totals) may be NULL. */
 int ifem_gpu_batch_init(ifem_gpu_ctx* ctx, int* neq, int64_t* nnz);
-/* One persistent launch over all (patch, node line) work items, largest
- * first: IFEM_GPU_FP64 writes K and b, IFEM_GPU_FP32 the FP32 copy of K. */
+/* One persistent launch per degree over its work items (groups of node lines
+ * of a patch, or segments of their rows), largest first: IFEM_GPU_FP64 writes
+ * K and b, IFEM_GPU_FP32 the FP32 copy of K. */
 int ifem_gpu_batch_assemble(ifem_gpu_ctx* ctx, int precision);
-/* Tunes, for each degree present (nen = (p+1)^3 element nodes), the element
- * chunk of the assembly (full or half) and the row entries per SpMV step
- * (16/32/64, two per lane) by timing the batch, then re-assembles with the choice.
+/* Tunes, for each degree present, the work split of the assembly (degrees 1
+ * and 2: row segments of full or half length, degree 3: full or half element
+ * chunks) and the row entries per SpMV step (16/32/64, two per lane) by timing
+ * the batch, then re-assembles with the choice.
  * table (may be NULL) receives 4 x {half, lanes} indexed by p. */
 int ifem_gpu_batch_autotune(ifem_gpu_ctx* ctx, int precision, int* table);
 /* Solves every patch to max(rtol*||b_q||, atol) on its true FP64 residual;
