@@ -1321,6 +1321,61 @@ int batch_upload_args(Context& c)
   return IFEM_GPU_OK;
 }
 
+// Work list of the line kernels: items are groups of neighbouring lines with a
+// segment of their rows (degree 3: whole lines), split so that every degree has
+// a few items per workgroup that the chip holds, largest first.  The second
+// list (half) has segments of half the length at degrees 1 and 2; it is built
+// when the tuner first asks for it.
+static int batch_items(Context& c, int half)
+{
+  Batch& B = *c.batch;
+  const int np = (int)B.pp.size();
+  struct Item { double cost; LineItem it; };
+  std::vector<LineItem> hi;
+  for (int p = half ? 2 : 3; p >= 1; p--) {
+    const int most = batch_lines_per_item(p);
+    int64_t groups = 0;
+    for (const BatchPatch& bp : B.pp) {
+      const PatchRec& Pt = c.patches[bp.patch];
+      if (bp.p == p && bp.neq > 0) groups += (int64_t)((Pt.n[1] + most - 1) / most) * Pt.n[2];
+    }
+    const int64_t want = groups > 0 ? (4 * B.ncu + groups - 1) / groups : 1; // segments per line
+    std::vector<Item> items;
+    for (int q = 0; q < np; q++) {
+      const BatchPatch& bp = B.pp[q];
+      if (bp.p != p || bp.neq == 0) continue;
+      const PatchRec& Pt = c.patches[bp.patch];
+      const int ngj = (Pt.n[1] + most - 1) / most;
+      int nseg = (int)std::min<int64_t>(want, std::max(1, Pt.n[0] / (4 * p)));
+      // few groups: down to one row each while every item has a compute
+      // unit (8 quadratic patches of 4 to 8 elements, FP32: 75 -> 55 us)
+      nseg = std::max(nseg, (int)std::min<int64_t>(Pt.n[0], B.ncu / groups));
+      if (half) nseg = std::min(2 * nseg, Pt.n[0]);
+      if (p == 3) nseg = 1; // whole lines (direct kernels)
+      for (int k = 0; k < Pt.n[2]; k++) {
+        const int c3 = std::min(k, Pt.nel[2] - 1) - std::max(0, k - p) + 1;
+        for (int g = 0; g < ngj; g++)
+          for (int sg = 0; sg < nseg; sg++) {
+            const int j0 = (int)((int64_t)Pt.n[1] * g / ngj), j1 = (int)((int64_t)Pt.n[1] * (g + 1) / ngj);
+            const int i0 = (int)((int64_t)Pt.n[0] * sg / nseg), i1 = (int)((int64_t)Pt.n[0] * (sg + 1) / nseg);
+            const int layers = std::min(i1, Pt.nel[0]) - std::max(0, i0 - p);
+            const int c2 = p == 3 ? std::min(j0, Pt.nel[1] - 1) - std::max(0, j0 - p) + 1 : 1;
+            items.push_back({(double)layers * c3 * c2, LineItem{q, j0, j1 - j0, k, i0, i1}});
+          }
+      }
+    }
+    std::stable_sort(items.begin(), items.end(),
+                     [](const Item& x, const Item& y) { return x.cost > y.cost; });
+    B.item0[half][p] = (int)hi.size();
+    for (const Item& it : items) hi.push_back(it.it);
+    B.item1[half][p] = (int)hi.size();
+  }
+  IFEM_HIP(hipMalloc(&B.d_items[half], sizeof(LineItem) * (hi.empty() ? 1 : hi.size())));
+  if (!hi.empty())
+    IFEM_HIP(hipMemcpy(B.d_items[half], hi.data(), sizeof(LineItem) * hi.size(), hipMemcpyHostToDevice));
+  return IFEM_GPU_OK;
+}
+
 // Symbolic phase of the batch: per-patch basis tables, global CSR pattern
 // (patch q's rows and columns are its equations shifted by eq0), and the
 // (patch, line) work list sorted by decreasing estimated cost.
@@ -1412,58 +1467,13 @@ int batch_symbolic(Context& c)
   IFEM_HIP(hipMemcpy(B.d_glist, glist.data(), sizeof(int) * glist.size(), hipMemcpyHostToDevice));
   IFEM_HIP(hipMemcpy(B.d_gq0, gq0.data(), sizeof(int64_t) * gq0.size(), hipMemcpyHostToDevice));
 
-  // work lists: items are groups of neighbouring lines with a segment of
-  // their rows, split so that every degree has a few items per workgroup that
-  // the chip holds; the second list has segments of half the length (tuning)
   hipDeviceProp_t prop;
   IFEM_HIP(hipGetDeviceProperties(&prop, c.device));
   B.ncu = prop.multiProcessorCount;
-  struct Item { double cost; LineItem it; };
-  std::vector<LineItem> hi;
-  for (int half = 0; half < 2; half++)
-    for (int p = 3; p >= 1; p--) {
-      const int most = batch_lines_per_item(p);
-      int64_t groups = 0;
-      for (const BatchPatch& bp : B.pp) {
-        const PatchRec& Pt = c.patches[bp.patch];
-        if (bp.p == p && bp.neq > 0) groups += (int64_t)((Pt.n[1] + most - 1) / most) * Pt.n[2];
-      }
-      const int64_t want = groups > 0 ? (4 * B.ncu + groups - 1) / groups : 1; // segments per line
-      std::vector<Item> items;
-      for (int q = 0; q < np; q++) {
-        const BatchPatch& bp = B.pp[q];
-        if (bp.p != p || bp.neq == 0) continue;
-        const PatchRec& Pt = c.patches[bp.patch];
-        const int ngj = (Pt.n[1] + most - 1) / most;
-        int nseg = (int)std::min<int64_t>(want, std::max(1, Pt.n[0] / (4 * p)));
-        // few groups: down to one row each while every item has a compute
-        // unit (8 quadratic patches of 4 to 8 elements, FP32: 75 -> 55 us)
-        nseg = std::max(nseg, (int)std::min<int64_t>(Pt.n[0], B.ncu / groups));
-        if (half) nseg = std::min(2 * nseg, Pt.n[0]);
-        if (p == 3) nseg = 1; // whole lines (direct kernels)
-        for (int k = 0; k < Pt.n[2]; k++) {
-          const int c3 = std::min(k, Pt.nel[2] - 1) - std::max(0, k - p) + 1;
-          for (int g = 0; g < ngj; g++)
-            for (int sg = 0; sg < nseg; sg++) {
-              const int j0 = (int)((int64_t)Pt.n[1] * g / ngj), j1 = (int)((int64_t)Pt.n[1] * (g + 1) / ngj);
-              const int i0 = (int)((int64_t)Pt.n[0] * sg / nseg), i1 = (int)((int64_t)Pt.n[0] * (sg + 1) / nseg);
-              const int layers = std::min(i1, Pt.nel[0]) - std::max(0, i0 - p);
-              const int c2 = p == 3 ? std::min(j0, Pt.nel[1] - 1) - std::max(0, j0 - p) + 1 : 1;
-              items.push_back({(double)layers * c3 * c2, LineItem{q, j0, j1 - j0, k, i0, i1}});
-            }
-        }
-      }
-      std::stable_sort(items.begin(), items.end(),
-                       [](const Item& x, const Item& y) { return x.cost > y.cost; });
-      B.item0[half][p] = (int)hi.size();
-      for (const Item& it : items) hi.push_back(it.it);
-      B.item1[half][p] = (int)hi.size();
-    }
-  IFEM_HIP(hipMalloc(&B.d_items, sizeof(LineItem) * (hi.empty() ? 1 : hi.size())));
-  if (!hi.empty())
-    IFEM_HIP(hipMemcpy(B.d_items, hi.data(), sizeof(LineItem) * hi.size(), hipMemcpyHostToDevice));
+  int rc = batch_items(c, 0);
+  if (rc) return rc;
   IFEM_HIP(hipMalloc(&B.d_queue, sizeof(int) * 4));
-  int rc = batch_upload_args(c);
+  rc = batch_upload_args(c);
   if (rc) return rc;
   IFEM_HIP(hipEventRecord(c.ev1, c.stream));
   IFEM_HIP(hipEventSynchronize(c.ev1));
@@ -1480,6 +1490,10 @@ int batch_assemble(Context& c, int precision, double* ms_out)
 {
   Batch& B = *c.batch;
   const bool fp32 = precision == IFEM_GPU_FP32;
+  if ((B.tune[1].half || B.tune[2].half) && !B.d_items[1]) {
+    const int rc = batch_items(c, 1);
+    if (rc) return rc;
+  }
   k_fill<int><<<1, 64, 0, c.stream>>>(4, B.d_queue, 0);
   IFEM_HIP(hipEventRecord(c.ev0, c.stream));
   // geometry pass: always for FP64 (the full assembly); an FP32 assembly
@@ -1501,10 +1515,10 @@ int batch_assemble(Context& c, int precision, double* ms_out)
     }
   }
   for (int p = 3; p >= 1; p--) {
-    const int half = B.tune[p].half ? 1 : 0;
+    const int half = p < 3 && B.tune[p].half ? 1 : 0;
     const int n = B.item1[half][p] - B.item0[half][p];
     if (n <= 0) continue;
-    const LineItem* items = static_cast<const LineItem*>(B.d_items) + B.item0[half][p];
+    const LineItem* items = static_cast<const LineItem*>(B.d_items[half]) + B.item0[half][p];
     const AsmArgs* args = static_cast<const AsmArgs*>(fp32 ? B.d_args32 : B.d_args64);
     const int rc = p == 3   ? launch_lines_batch3(c, args, items, n, B.d_queue + p, B.ncu, fp32)
                    : p == 2 ? launch_lines_batch2(c, args, items, n, B.d_queue + p, B.ncu, fp32)

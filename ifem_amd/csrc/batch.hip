@@ -282,7 +282,7 @@ void Batch::release()
   }
   pp.clear();
   void** d[] = {(void**)&d_rowptr, (void**)&d_colind, (void**)&d_val, (void**)&d_val32,
-                (void**)&d_rhs, &d_args64, &d_args32, (void**)&d_items, (void**)&d_queue,
+                (void**)&d_rhs, &d_args64, &d_args32, &d_items[0], &d_items[1], (void**)&d_queue,
                 (void**)&d_crow0, (void**)&d_cpatch, (void**)&d_clanes, (void**)&d_pchunk,
                 (void**)&x, (void**)&r, (void**)&z, (void**)&p, (void**)&q, (void**)&dinv,
                 (void**)&r32, (void**)&z32, (void**)&p32, (void**)&q32, (void**)&x32,

@@ -64,7 +64,8 @@ struct Batch {
   // assembly work list and per-patch arguments (AsmArgs, FP64 and FP32)
   void* d_args64 = nullptr;
   void* d_args32 = nullptr;
-  void* d_items = nullptr; // LineItem; of degree p in list h: [item0[h][p], item1[h][p])
+  // lists of LineItem (batch_items); of degree p in list h: [item0[h][p], item1[h][p])
+  void* d_items[2] = {nullptr, nullptr};
   int item0[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}}, item1[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
   int* d_queue = nullptr;   // one queue counter per degree
   int ncu = 0;              // compute units (persistent grid size)
