@@ -668,7 +668,7 @@ int ifem_gpu_spmv_noalloc(ifem_gpu_ctx* ctx, const double* x, double* y)
   double* dy = c.noalloc_scratch + kNoAllocMaxEq;
   if (hipMemcpyAsync(dx, x, sizeof(double) * c.neq, hipMemcpyHostToDevice, c.stream) != hipSuccess)
     return fail(IFEM_GPU_EDEVICE, "spmv_noalloc: copy in failed");
-  int rc = spmv_device(c, dx, dy, false);
+  int rc = spmv_device(c, dx, dy);
   if (!rc && hipMemcpyAsync(y, dy, sizeof(double) * c.neq, hipMemcpyDeviceToHost, c.stream) != hipSuccess)
     rc = fail(IFEM_GPU_EDEVICE, "spmv_noalloc: copy out failed");
   if (!rc && hipStreamSynchronize(c.stream) != hipSuccess)

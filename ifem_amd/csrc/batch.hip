@@ -373,15 +373,10 @@ static int batch_solver_setup(Context& c)
   B.iters.assign(np, 0);
   B.conv.assign(np, 0);
   B.relres.assign(np, 0.0);
+  rc = build_row_shapes(c.stream, B.neq, B.d_rowptr, B.d_colind, false, B.nnz, B.shapes);
+  if (rc) return rc;
   IFEM_HIP(hipStreamSynchronize(c.stream));
   return IFEM_GPU_OK;
-}
-
-// Row shapes of the batch, before its first product.
-static int batch_shapes(Context& c)
-{
-  Batch& B = *c.batch;
-  return find_row_shapes(c.stream, B.neq, B.d_rowptr, B.d_colind, false, B.nnz, B.shapes);
 }
 
 template <typename V, typename ACC, bool DOT>
@@ -520,10 +515,8 @@ int batch_solve(Context& c, const ifem_gpu_solver_params& prm, ifem_gpu_stats* s
   const int n = B.neq;
   const int nb = (n + 255) / 256;
   IFEM_HIP(hipEventRecord(c.ev0, c.stream));
-  int rc = batch_shapes(c); // before the iterations are captured
-  if (rc) return rc;
   std::vector<double> bb;
-  rc = batch_norms(c, nullptr, B.r, bb); // r = b
+  int rc = batch_norms(c, nullptr, B.r, bb); // r = b
   if (rc) return rc;
   std::vector<double> bnorm(np), tol(np), rr(np);
   std::vector<int> state(np, 0); // 0 iterating, 1 converged, 2 stopped
@@ -675,8 +668,6 @@ int batch_autotune(Context& c, int precision, int* table)
     rc = batch_assemble(c, IFEM_GPU_FP32, nullptr);
     if (rc) return rc;
   }
-  rc = batch_shapes(c);
-  if (rc) return rc;
   const int lanes_c[3] = {16, 32, 64};
   for (int p = 1; p <= 3; p++) {
     if (!present[p]) continue;

@@ -26,12 +26,10 @@ struct BatchPatch {
 };
 
 // Row shapes of a sparsity pattern (shapes.hip): row r's k-th column is
-// r + table[start[r] + k]; start == nullptr: not available.  Searched for by
-// the pattern's first product or solve (searched).
+// r + table[start[r] + k]; start == nullptr: not available.
 struct RowShapes {
   int32_t* start = nullptr;
   int32_t* table = nullptr;
-  bool searched = false;
   void release();
 };
 

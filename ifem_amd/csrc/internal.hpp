@@ -240,16 +240,14 @@ int batch_solve(Context& c, const ifem_gpu_solver_params& prm, ifem_gpu_stats* s
 int batch_autotune(Context& c, int precision, int* table);
 
 // shapes.hip: row shapes of n rows (nodal: node triples, cols = node columns,
-// rowptr per equation) with `entries` column indices in all, on the first call
-// for a pattern outside of a stream capture (the search allocates and waits)
-int find_row_shapes(hipStream_t s, int n, const int64_t* rowptr, const int32_t* cols, bool nodal,
+// rowptr per equation) with `entries` column indices in all
+int build_row_shapes(hipStream_t s, int n, const int64_t* rowptr, const int32_t* cols, bool nodal,
                      int64_t entries, RowShapes& out);
 
 // solver.hip
 int solver_setup(Context& c);
 int solve(Context& c, const ifem_gpu_solver_params& prm, ifem_gpu_stats* st);
-int system_shapes(Context& c);
-int spmv_device(Context& c, const double* d_x, double* d_y, bool may_allocate = true);
+int spmv_device(Context& c, const double* d_x, double* d_y);
 int spmv_device32(Context& c, const float* d_x, float* d_y);
 void solver_free(Context& c);
 int set_learned(Context& c, int enable, int D, int H, int W, const float* aux, int naux,

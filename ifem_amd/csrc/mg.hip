@@ -1038,7 +1038,6 @@ int mg_setup(Context& c, int degree)
   Multigrid& m = *c.mg;
   m.degree = degree;
   IFEM_HIP(hipEventRecord(m.e0, c.stream));
-  if (const int rc = system_shapes(c)) return rc;
   // fine level: inverse diagonal, then K / max diag in FP16 for the smoother
   MgLevel& F = m.lev[0];
   k_mg_diag<<<kMgParts, kThreads, 0, c.stream>>>(c.neq, c.d_rowptr, c.d_colind, c.d_val, F.dinv,

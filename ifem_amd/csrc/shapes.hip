@@ -179,18 +179,15 @@ static int build(hipStream_t s, int n, const ShapeRows& R, int64_t entries, RowS
   return IFEM_GPU_OK;
 }
 
-int find_row_shapes(hipStream_t s, int n, const int64_t* rowptr, const int32_t* cols, bool nodal,
-                    int64_t entries, RowShapes& out)
+int build_row_shapes(hipStream_t s, int n, const int64_t* rowptr, const int32_t* cols, bool nodal,
+                     int64_t entries, RowShapes& out)
 {
-  if (out.searched || n <= 0 || entries <= 0) return IFEM_GPU_OK;
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  IFEM_HIP(hipStreamIsCapturing(s, &capture));
-  if (capture != hipStreamCaptureStatusNone) return IFEM_GPU_OK;
+  out.release();
+  if (n <= 0 || entries <= 0) return IFEM_GPU_OK;
   void* tmp[4] = {};
   const int rc = build(s, n, ShapeRows{rowptr, cols, nodal ? 1 : 0}, entries, out, tmp);
   for (void* t : tmp) hipFree(t);
   if (rc) out.release();
-  out.searched = rc == IFEM_GPU_OK;
   return rc;
 }
 
@@ -199,7 +196,6 @@ void RowShapes::release()
   hipFree(start);
   hipFree(table);
   start = table = nullptr;
-  searched = false;
 }
 
 } // namespace ifem

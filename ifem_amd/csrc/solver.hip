@@ -531,21 +531,9 @@ void launch_spmv16_node3(Context& c, const uint2* val, float scale, const float*
               : run(k_spmv_node3_h<false, false>, nullptr, c.d_bcol);
 }
 
-// Row shapes of the bound system, before its first product.
-int system_shapes(Context& c)
-{
-  const bool nodal = c.d_bcol != nullptr;
-  return find_row_shapes(c.stream, nodal ? c.neq / 3 : c.neq, c.d_rowptr,
-                         nodal ? c.d_bcol : c.d_colind, nodal, nodal ? c.nnz / 9 : c.nnz, c.shapes);
-}
-
-int spmv_device(Context& c, const double* d_x, double* d_y, bool may_allocate)
+int spmv_device(Context& c, const double* d_x, double* d_y)
 {
   if (c.neq == 0) return IFEM_GPU_OK;
-  if (may_allocate) {
-    const int rc = system_shapes(c);
-    if (rc) return rc;
-  }
   launch_spmv<double, double, false>(c, c.d_val, d_x, d_y);
   IFEM_HIP(hipGetLastError());
   return IFEM_GPU_OK;
@@ -554,8 +542,6 @@ int spmv_device(Context& c, const double* d_x, double* d_y, bool may_allocate)
 int spmv_device32(Context& c, const float* d_x, float* d_y)
 {
   if (c.neq == 0) return IFEM_GPU_OK;
-  const int rc = system_shapes(c);
-  if (rc) return rc;
   launch_spmv<float, float, false>(c, c.d_val32, d_x, d_y);
   IFEM_HIP(hipGetLastError());
   return IFEM_GPU_OK;
@@ -600,7 +586,10 @@ int solver_setup(Context& c)
     k_build_bcol<<<c.neq / 3, 128, 0, c.stream>>>(c.neq / 3, c.d_rowptr, c.d_colind, c.d_bcol);
     IFEM_HIP(hipGetLastError());
   }
-  c.shapes.release(); // of the pattern before
+  int rc = build_row_shapes(c.stream, uniform ? c.neq / 3 : c.neq, c.d_rowptr,
+                            uniform ? c.d_bcol : c.d_colind, uniform,
+                            uniform ? c.nnz / 9 : c.nnz, c.shapes);
+  if (rc) return rc;
   w.nblocks = kGrid;
   IFEM_HIP(hipStreamSynchronize(c.stream));
   return IFEM_GPU_OK;
@@ -1100,8 +1089,6 @@ int solve(Context& c, const ifem_gpu_solver_params& prm, ifem_gpu_stats* st)
   const int check = prm.check_every > 0 ? prm.check_every : 32;
   int rc;
   IFEM_HIP(hipEventRecord(c.ev0, c.stream));
-  rc = system_shapes(c);
-  if (rc) return rc;
   double bb = 0.0;
   rc = norm2_rhs(c, &bb);
   if (rc) return rc;

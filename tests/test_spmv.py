@@ -127,11 +127,10 @@ def _hip(name, *args):
     assert rc == 0, (name, rc)
 
 
-def test_row_shapes_come_with_the_first_product():
-    """The search for row shapes is the first product's, not the set-up's, so
-    every way to make that product has to give the same bits: recorded in a
-    graph (no search can be made there), without allocation, plain, and after a
-    system of another pattern in the same session."""
+def test_first_products_of_every_kind():
+    """The first product of a system gives the same bits whichever way it is
+    made: plain, without allocation, recorded in a graph, and in a session that
+    held a system of another pattern before."""
     def bind(s, nel, p):
         P = M.cube_patch(p, list(nel), 0.1, seed=p)
         meqn, neq = M.equation_numbers(M.face_status(P, 1, [0] * 6))
