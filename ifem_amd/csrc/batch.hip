@@ -373,7 +373,8 @@ static int batch_solver_setup(Context& c)
   B.iters.assign(np, 0);
   B.conv.assign(np, 0);
   B.relres.assign(np, 0.0);
-  rc = build_row_shapes(c.stream, B.neq, B.d_rowptr, B.d_colind, false, B.nnz, B.shapes);
+  rc = build_row_shapes(c.stream, B.neq, B.d_rowptr, B.d_colind, false, B.nnz, B.d_val,
+                        sizeof(double) * B.nnz, B.shapes);
   if (rc) return rc;
   IFEM_HIP(hipStreamSynchronize(c.stream));
   return IFEM_GPU_OK;

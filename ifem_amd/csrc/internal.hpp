@@ -240,9 +240,10 @@ int batch_solve(Context& c, const ifem_gpu_solver_params& prm, ifem_gpu_stats* s
 int batch_autotune(Context& c, int precision, int* table);
 
 // shapes.hip: row shapes of n rows (nodal: node triples, cols = node columns,
-// rowptr per equation) with `entries` column indices in all
+// rowptr per equation) with `entries` column indices in all; work: device
+// memory that holds nothing yet (the values), used instead of an allocation
 int build_row_shapes(hipStream_t s, int n, const int64_t* rowptr, const int32_t* cols, bool nodal,
-                     int64_t entries, RowShapes& out);
+                     int64_t entries, void* work, size_t work_bytes, RowShapes& out);
 
 // solver.hip
 int solver_setup(Context& c);

@@ -10,7 +10,10 @@
 // compared with its shape's list entry by entry, and any difference (a hash
 // collision) drops the shapes.  Patterns whose lists are mostly distinct
 // (fixed DOFs strewn over the patch) keep their column indices: the table must
-// be at most an eighth of them.
+// be at most an eighth of them.  So do small systems, whose products read the
+// indices from the caches as fast (cubes of linear scalar elements, FP64: 28^3
+// 4.4 us with shapes, 3.4 without; 40^3 4.9 and 5.1; 90^3 36.6 and 46.6): there
+// the search would be up to nine tenths of a pattern's set-up.
 #include <hip/hip_runtime.h>
 
 #include <rocprim/device/device_radix_sort.hpp>
@@ -125,38 +128,35 @@ __global__ void k_shape_check(ShapeRows R, int n, int total, const int32_t* __re
 __global__ void k_shape_clear(int* bad) { *bad = 0; }
 
 static int build(hipStream_t s, int n, const ShapeRows& R, int64_t entries, RowShapes& out,
-                 void* (&tmp)[4])
+                 void* work, size_t work_bytes, void*& tmp)
 {
-  uint64_t *key = nullptr, *skey = nullptr;
-  int *row = nullptr, *srow = nullptr, *head = nullptr, *len = nullptr;
-  int64_t* incl = nullptr;
+  size_t tb = 0, tb2 = 0;
+  IFEM_HIP(rocprim::radix_sort_pairs(nullptr, tb, (uint64_t*)nullptr, (uint64_t*)nullptr, (int*)nullptr,
+                                     (int*)nullptr, (size_t)n, 0, 64, s));
+  IFEM_HIP(rocprim::inclusive_scan(nullptr, tb2, (int*)nullptr, (int64_t*)nullptr, (size_t)n,
+                                   rocprim::plus<int64_t>(), s));
+  if (tb2 > tb) tb = tb2;
   // without memory for the search the products keep the column indices
   auto alloc = [](void** p, size_t bytes) {
     if (hipMalloc(p, bytes) == hipSuccess) return true;
     (void)hipGetLastError();
     return false;
   };
-  if (!alloc(&tmp[0], sizeof(uint64_t) * 2 * (size_t)n) ||
-      !alloc(&tmp[1], sizeof(int) * 4 * (size_t)n) ||
-      !alloc(&tmp[2], sizeof(int64_t) * ((size_t)n + 1)))
-    return IFEM_GPU_OK;
-  key = static_cast<uint64_t*>(tmp[0]);
-  skey = key + n;
-  row = static_cast<int*>(tmp[1]);
-  srow = row + n;
-  head = srow + n;
-  len = head + n;
-  incl = static_cast<int64_t*>(tmp[2]);
-  int* bad = reinterpret_cast<int*>(incl + n);
+  const size_t rows = (size_t)n, head_bytes = 40 * rows + 16, need = (head_bytes + 255) / 256 * 256 + tb;
+  if (need > work_bytes) {
+    if (!alloc(&tmp, need)) return IFEM_GPU_OK;
+    work = tmp;
+  }
+  uint64_t *key = static_cast<uint64_t*>(work), *skey = key + n;
+  int64_t* incl = reinterpret_cast<int64_t*>(skey + n);
+  int* bad = reinterpret_cast<int*>(incl + n); // two words
+  int *row = bad + 2, *srow = row + n, *head = srow + n, *len = head + n;
+  void* sort_tmp = static_cast<char*>(work) + (head_bytes + 255) / 256 * 256;
   const unsigned nb = (unsigned)((n + 255) / 256), nwv = (unsigned)((n + 3) / 4 < 8192 ? (n + 3) / 4 : 8192);
   k_shape_hash<<<nwv, 256, 0, s>>>(R, n, key, row);
-  size_t tb = 0, tb2 = 0;
-  IFEM_HIP(rocprim::radix_sort_pairs(nullptr, tb, key, skey, row, srow, (size_t)n, 0, 64, s));
-  IFEM_HIP(rocprim::inclusive_scan(nullptr, tb2, len, incl, (size_t)n, rocprim::plus<int64_t>(), s));
-  if (!alloc(&tmp[3], tb > tb2 ? tb : tb2)) return IFEM_GPU_OK;
-  IFEM_HIP(rocprim::radix_sort_pairs(tmp[3], tb, key, skey, row, srow, (size_t)n, 0, 64, s));
+  IFEM_HIP(rocprim::radix_sort_pairs(sort_tmp, tb, key, skey, row, srow, (size_t)n, 0, 64, s));
   k_shape_heads<<<nb, 256, 0, s>>>(R, n, skey, srow, head, len);
-  IFEM_HIP(rocprim::inclusive_scan(tmp[3], tb2, len, incl, (size_t)n, rocprim::plus<int64_t>(), s));
+  IFEM_HIP(rocprim::inclusive_scan(sort_tmp, tb, len, incl, (size_t)n, rocprim::plus<int64_t>(), s));
   int64_t total = 0;
   IFEM_HIP(hipMemcpyAsync(&total, incl + n - 1, sizeof(int64_t), hipMemcpyDeviceToHost, s));
   IFEM_HIP(hipStreamSynchronize(s));
@@ -179,14 +179,18 @@ static int build(hipStream_t s, int n, const ShapeRows& R, int64_t entries, RowS
   return IFEM_GPU_OK;
 }
 
+// Column indices that the products read from the caches as fast as row shapes:
+// 4 MB, an XCD's L2.
+constexpr int64_t kMinEntries = 1 << 20;
+
 int build_row_shapes(hipStream_t s, int n, const int64_t* rowptr, const int32_t* cols, bool nodal,
-                     int64_t entries, RowShapes& out)
+                     int64_t entries, void* work, size_t work_bytes, RowShapes& out)
 {
   out.release();
-  if (n <= 0 || entries <= 0) return IFEM_GPU_OK;
-  void* tmp[4] = {};
-  const int rc = build(s, n, ShapeRows{rowptr, cols, nodal ? 1 : 0}, entries, out, tmp);
-  for (void* t : tmp) hipFree(t);
+  if (n <= 0 || entries < kMinEntries) return IFEM_GPU_OK;
+  void* tmp = nullptr;
+  const int rc = build(s, n, ShapeRows{rowptr, cols, nodal ? 1 : 0}, entries, out, work, work_bytes, tmp);
+  hipFree(tmp);
   if (rc) out.release();
   return rc;
 }

@@ -588,7 +588,7 @@ int solver_setup(Context& c)
   }
   int rc = build_row_shapes(c.stream, uniform ? c.neq / 3 : c.neq, c.d_rowptr,
                             uniform ? c.d_bcol : c.d_colind, uniform,
-                            uniform ? c.nnz / 9 : c.nnz, c.shapes);
+                            uniform ? c.nnz / 9 : c.nnz, c.d_val, sizeof(double) * c.nnz, c.shapes);
   if (rc) return rc;
   w.nblocks = kGrid;
   IFEM_HIP(hipStreamSynchronize(c.stream));

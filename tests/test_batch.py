@@ -120,9 +120,9 @@ def test_batch_mixed_precision_and_autotune():
 
 
 def test_batch_with_row_shapes_and_row_segments():
-    """Patches large enough for the product to read row shapes (distinct lists
-    of column offsets at most an eighth of all; the small batches above read
-    column indices) and few enough for lines to be cut into row segments: K and
+    """Patches large enough for the product to read row shapes (2^20 column
+    indices, distinct lists at most an eighth of them; the small batches above
+    read column indices) and few enough for lines to be cut into row segments: K and
     b against the oracle, solutions by the host's residual and energy norm."""
     pbs = problems.diffusion_batch(6, (12, 16), (1, 2, 3), sigma=1.0, ell=0.2, seed=9, nmodes=32)
     degrees = [pb.patch.p[0] for pb in pbs]
@@ -141,7 +141,7 @@ def test_batch_with_row_shapes_and_row_segments():
             lists += sum({(ci[rp[r]:rp[r + 1]] - r).tobytes(): rp[r + 1] - rp[r]
                           for r in range(pb.neq)}.values())
             entries += len(ci)
-        assert lists <= entries // 8
+        assert entries >= 1 << 20 and lists <= entries // 8
         st = s.batch_solve(rtol=1e-12, maxits=5000)
         x64 = [s.batch_solution(k) for k in range(len(pbs))]
         assert st["converged"]

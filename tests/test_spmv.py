@@ -1,8 +1,8 @@
 """Matrix-vector products (GPU) over the row layouts they tell apart: scalar
-rows and node triples, columns from row shapes (free or face-fixed patches that
-are large enough for their lists to repeat) and from the column indices (small
-patches, fixings strewn over the patch), rows shorter and longer than a round
-of their lanes, each number of lanes.
+rows and node triples, columns from row shapes (free or face-fixed patches of
+at least 2^20 column indices) and from the column indices (smaller patches,
+fixings strewn over the patch), rows shorter and longer than a round of their
+lanes, each number of lanes.
 
 A sum of n products is within n units of roundoff of its exact value, relative
 to the sum of the absolute products; rows hold at most 1029 entries and both
@@ -50,8 +50,9 @@ def test_product_of_every_row_layout(nc, p, nel, fix):
 
 
 def _shapes_kept(rp, ci, nodal):
-    """Whether the distinct lists of column offsets take at most an eighth of
-    the (node) column indices: the products then read the lists."""
+    """Whether there are at least 2^20 (node) column indices and the distinct
+    lists of column offsets take at most an eighth of them: the products then
+    read the lists."""
     if nodal:
         n = (len(rp) - 1) // 3
         cnt = np.diff(rp)[::3] // 3
@@ -60,15 +61,15 @@ def _shapes_kept(rp, ci, nodal):
     else:
         n, start = len(rp) - 1, rp
     lists = {(ci[start[r]:start[r + 1]] - r).tobytes() for r in range(n)}
-    return sum(map(len, lists)) // ci.itemsize <= start[-1] // 8
+    return start[-1] >= 1 << 20 and sum(map(len, lists)) // ci.itemsize <= start[-1] // 8
 
 
 # lanes: of the rows or nodes of this size (4 or 16: short lists; 32 or 64: long
 # lists of few rows; 8 or 32: others)
 @pytest.mark.parametrize("nc,p,nel,lanes", [
-    (1, 1, (16, 9, 8), 4), (1, 2, (12, 10, 11), 8), (1, 3, (12, 11, 13), 32),
-    (1, 3, (30, 26, 24), 8), (3, 1, (14, 9, 8), 16), (3, 2, (12, 10, 11), 32),
-    (3, 3, (13, 11, 12), 64), (3, 3, (150, 20, 2), 32)])
+    (1, 1, (48, 36, 31), 4), (1, 2, (25, 23, 22), 8), (1, 3, (22, 21, 20), 32),
+    (1, 3, (30, 26, 24), 8), (3, 1, (37, 33, 34), 16), (3, 2, (24, 21, 22), 32),
+    (3, 3, (18, 15, 16), 64), (3, 3, (150, 20, 2), 32)])
 def test_products_from_row_shapes(nc, p, nel, lanes):
     P = M.cube_patch(p, list(nel), 0.1, seed=p + nc)
     fix = [7, 0, 0, 7, 0, 0] if nc == 3 else [0] * 6
